@@ -91,7 +91,7 @@ __device__ inline DevField frame_field(const BatchDev &b, int f) {
 }
 
 /* one particle, at most `budget` steps; returns with its state stored */
-template <int MODE, int GEN>
+template <int MODE, int GEN, int BS>
 __device__ void batch_particle(const DevMesh &m, const BatchDev &b, int i, int budget, uint32_t &ns) {
 #pragma clang fp contract(off)
     int fl = b.flags[i];
@@ -142,7 +142,8 @@ __device__ void batch_particle(const DevMesh &m, const BatchDev &b, int i, int b
         const uint32_t before = ns;
         double stop;
         const int finished =
-            interval_run<MODE, 3, 1, GEN>(m, fld, s, is, ia, ib, b.dt, R.itype, 0, left_budget, err, ns, stop);
+            interval_run<MODE, 3, 1, GEN>(m, fld, s, is, ia, ib, b.dt, R.itype, 0, left_budget, err, ns, stop,
+                                        sm_rows<MODE, 3, 1, GEN, BS>());
         if (err) break;
         if (!finished) { /* budget spent inside the interval */
             fl |= FL_STARTED;
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(GEN ? 2 : FV
             const int base = claim64(&b.queue[q], seg_hi - seg_lo);
             if (seg_lo + base >= seg_hi) break;
             const int idx = seg_lo + base + lane;
-            if (idx < seg_hi) batch_particle<MODE, GEN>(m, b, b.list_in[idx], budget, ns);
+            if (idx < seg_hi) batch_particle<MODE, GEN, BS>(m, b, b.list_in[idx], budget, ns);
         }
     }
     unsigned long long v = ns;

@@ -265,15 +265,20 @@ __device__ __forceinline__ void nat_fast(const DevMesh &m, int e, double x, doub
 
 /* query anchored in FP32: the point (centre + A) + d, q - o = (A - o) + d */
 template <int DIM>
-__device__ __forceinline__ void nat_fast_c(const DevMesh &m, int e, const float A[3], const float d[3], float &r,
-                                           float &s, float &t, float &ge) {
+__device__ __forceinline__ void nat_frame(const Frame &F, const float A[3], const float d[3], float &r, float &s,
+                                          float &t, float &ge) {
 #pragma clang fp contract(off)
-    const Frame F = ld_frame<DIM>(m, e);
     const float qx = (A[0] - F.a0.w) + d[0];
     const float qy = (A[1] - F.a1.w) + d[1];
     const float qz = DIM == 3 ? (A[2] - F.a2.w) + d[2] : 0.0f;
     frame_nat<DIM>(F, qx, qy, qz, r, s, t);
     ge = F.a3.w;
+}
+
+template <int DIM>
+__device__ __forceinline__ void nat_fast_c(const DevMesh &m, int e, const float A[3], const float d[3], float &r,
+                                           float &s, float &t, float &ge) {
+    nat_frame<DIM>(ld_frame<DIM>(m, e), A, d, r, s, t, ge);
 }
 
 /* guard term of a query offset d (its rounding in (A - o) + d) */
@@ -286,26 +291,28 @@ __device__ __forceinline__ float guard_offset(const DevMesh &m, const float d[3]
 template <int DIM>
 __device__ __forceinline__ int decide_fast(float r, float s, float t, float ge, float gq, int &slot) {
 #pragma clang fp contract(off)
-    float l0 = DIM == 3 ? ((1.0f - r) - s) - t : (1.0f - r) - s;
-    float v[4] = {r, s, DIM == 3 ? t : l0, l0};
-    const int n = DIM == 3 ? 4 : 3;
-    int a = 0;
-    float d = v[0], L = fabsf(v[0]);
-    for (int q = 1; q < n; q++) {
-        L = fmaxf(L, fabsf(v[q]));
-        if (v[q] < d) {
-            d = v[q];
-            a = q;
-        }
-    }
+    const float l0 = DIM == 3 ? ((1.0f - r) - s) - t : (1.0f - r) - s;
+    /* smallest and second smallest by pairs, without arrays (a dynamically
+     * indexed array would go through LDS) */
+    const float lo1 = fminf(r, s), hi1 = fmaxf(r, s);
+    const float lo2 = DIM == 3 ? fminf(t, l0) : l0, hi2 = DIM == 3 ? fmaxf(t, l0) : 3.0e38f;
+    const float d = fminf(lo1, lo2);
+    const float L = fmaxf(fmaxf(fabsf(r), fabsf(s)), DIM == 3 ? fmaxf(fabsf(t), fabsf(l0)) : fabsf(l0));
     const float g = __builtin_fmaf(ge, fmaxf(L, 1.0f), gq);
-    if (d > g) return 1;
+    const bool num = r == r; /* a query that is not a number moves on through slot 0 */
+    if (d > g && num) return 1;
+    slot = 0;
+    if (!num) return 0;
     if (d >= -g) return 2;
-    float second = 3.0e38f;
-    for (int q = 0; q < n; q++)
-        if (q != a && v[q] < second) second = v[q];
+    const float second = fminf(fmaxf(lo1, lo2), fminf(hi1, hi2));
     if (second - d <= 2.0f * g) return 2;
-    slot = a;
+    if (s == d) slot = 1;
+    if (DIM == 3) {
+        if (t == d) slot = 2;
+        if (l0 == d) slot = 3;
+    } else if (l0 == d) {
+        slot = 2;
+    }
     return 0;
 }
 
@@ -1140,10 +1147,93 @@ __device__ inline double strain_rate(const DevMesh &m, const DevField &f, double
  * double position X, a probe's at (centre + A) + d. */
 enum { PH_F0 = 0, PH_K2 = 1, PH_K3 = 2, PH_K4 = 3, PH_LOC = 4, PH_DONE = 5 };
 
+/* Per-lane rows of LDS holding the frame of the element a lane tested last
+ * and the node velocities (both slices) of the element it interpolated in
+ * last; row k of lane l is at [64 k + l], so a wave's 16-byte accesses are
+ * contiguous.
+ * Why: gathered anew, a pass costs 13 per-lane gathers (frame, connectivity,
+ * eight node velocities), and their tag look-ups kept the L1 busy 94% of the
+ * cycles (1.1-1.2 look-ups per CU and cycle, 32 per particle-step) with the
+ * vector ALUs at 64-68%; but a probe moves a tenth of an element per step, so
+ * nearly every pass asks for what the lane had in the pass before.  With the
+ * rows only lanes whose element changed gather: 5.8 look-ups per step, vector
+ * ALUs 72-79% busy.  k_advect (4M tracers, 20 steps, 5.6M tets) 3.44 -> 2.76
+ * ms a launch, k_ftle_advect (96x96x480 points) 4.49 -> 2.66 ms, the RK4
+ * class of a batch 2.1 -> 1.2 ms.  LDS and not registers: held in registers
+ * (40 more) the kernels spill 56-64 at 4 waves per SIMD.  160 bytes a lane
+ * in FP32 is the whole LDS at 4 waves per SIMD (16 waves of 10 KB), which is
+ * why nothing else of these kernels lies there. */
+template <int MODE, int DIM>
+struct SmRows {
+    static constexpr int NN = DIM == 3 ? 4 : 3;
+    static constexpr int FRAME = DIM == 3 ? 4 : 3;
+    static constexpr int VEL = (NN * (MODE == P_F32 ? 6 : 4) + 3) / 4;
+    static constexpr int N = MODE == P_F64 ? 0 : FRAME + VEL;
+};
+
+/* this lane's rows in a block of BS lanes (null in the kernels that do not
+ * run the state machine) */
+template <int MODE, int DIM, int UNS, int GEN, int BS>
+__device__ __forceinline__ float4 *sm_rows() {
+    constexpr int N = UNS && !GEN ? SmRows<MODE, DIM>::N : 0;
+    if constexpr (N > 0) {
+        __shared__ float4 s_rows[N * BS];
+        return s_rows + (threadIdx.x >> 6) * (64 * N) + (threadIdx.x & 63);
+    } else {
+        return nullptr;
+    }
+}
+
+template <int MODE, int DIM>
+__device__ __forceinline__ void vel_to_rows(const NodeVel<MODE, DIM> &g, float4 *rows) {
+    constexpr int NN = NodeVel<MODE, DIM>::NN, W = MODE == P_F32 ? 6 : 4;
+    float w[4 * SmRows<MODE, DIM>::VEL] = {};
+    for (int q = 0; q < NN; q++) {
+        if constexpr (MODE == P_F32) {
+            w[W * q] = g.lo[q].x;
+            w[W * q + 1] = g.lo[q].y;
+            w[W * q + 2] = g.lo[q].z;
+            w[W * q + 3] = g.hi[q].x;
+            w[W * q + 4] = g.hi[q].y;
+            w[W * q + 5] = g.hi[q].z;
+        } else {
+            w[W * q] = __uint_as_float(g.lo[q].x);
+            w[W * q + 1] = __uint_as_float(g.lo[q].y);
+            w[W * q + 2] = __uint_as_float(g.hi[q].x);
+            w[W * q + 3] = __uint_as_float(g.hi[q].y);
+        }
+    }
+    for (int k = 0; k < SmRows<MODE, DIM>::VEL; k++)
+        rows[64 * k] = make_float4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+}
+
+template <int MODE, int DIM>
+__device__ __forceinline__ void vel_from_rows(const float4 *rows, NodeVel<MODE, DIM> &g) {
+    constexpr int NN = NodeVel<MODE, DIM>::NN, W = MODE == P_F32 ? 6 : 4;
+    float w[4 * SmRows<MODE, DIM>::VEL];
+    for (int k = 0; k < SmRows<MODE, DIM>::VEL; k++) {
+        const float4 v = rows[64 * k];
+        w[4 * k] = v.x;
+        w[4 * k + 1] = v.y;
+        w[4 * k + 2] = v.z;
+        w[4 * k + 3] = v.w;
+    }
+    for (int q = 0; q < NN; q++) {
+        if constexpr (MODE == P_F32) {
+            g.lo[q] = F3{w[W * q], w[W * q + 1], w[W * q + 2]};
+            g.hi[q] = F3{w[W * q + 3], w[W * q + 4], w[W * q + 5]};
+        } else {
+            g.lo[q] = make_uint2(__float_as_uint(w[W * q]), __float_as_uint(w[W * q + 1]));
+            g.hi[q] = make_uint2(__float_as_uint(w[W * q + 2]), __float_as_uint(w[W * q + 3]));
+        }
+    }
+}
+
 template <int MODE, int DIM>
 __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is, double a, double b, double dt,
-                      int max_steps, int &err, uint32_t &nsteps, double &stop) {
+                      int max_steps, int &err, uint32_t &nsteps, double &stop, float4 *rows) {
 #pragma clang fp contract(off)
+    using R = SmRows<MODE, DIM>;
     if (!is.started) {
         if (p.left) {
             err = E_LEFT;
@@ -1166,34 +1256,26 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
     const double hmin = 1e-12 * fabs(dt);
     const double inv_span = 1.0 / (f.tmax - f.tmin);
     int taken = 0, ret = 1;
-    int phase = PH_F0, e = 0, hops = 0, start = 0;
+    int phase = PH_F0, hops = 0;
+    bool tie = false;  /* a test of this locate walk hit d == -TINY */
+    bool gone = false; /* a probe of this step left the mesh */
+    /* the probes' elements, a ring: q0 is the walk start of the probe whose
+     * turn it is (at a step's start and in the locate walk the first stage's) */
+    int q0 = is.mp[0].elem, q1 = is.mp[1].elem, q2 = is.mp[2].elem, q3 = is.mp[3].elem;
     /* S: f0, then f0 + 2 k2, f0 + 2 k2 + 2 k3, and from the k4 stage to the
      * locate's end the step's f0 + 2 k2 + 2 k3 + k4 (increment h/6 S) */
-    float A[3], D[3], dq[3], S[3] = {0.f, 0.f, 0.f};
-    float gD = 0.f, gdq = 0.f; /* guard terms of the offsets D and dq */
-    /* anchors of X: A = (float)(X - centre), D its FP32 residual */
+    float A[3], D[3], c[3], S[3] = {0.f, 0.f, 0.f}, gc;
+    float tl0 = 0.f, tlh = 0.f, tl1 = 0.f; /* time locations of the step's start, middle and end */
+    /* anchors of X: A = (float)(X - centre), D its FP32 residual; the walk at
+     * X has the offset c = D */
     auto anchor = [&]() {
-        for (int c = 0; c < 3; c++) {
-            const double xc = p.X[c] - m.centre[c];
-            A[c] = (float)xc;
-            D[c] = (float)(xc - (double)A[c]);
+        for (int k = 0; k < 3; k++) {
+            const double xc = p.X[k] - m.centre[k];
+            A[k] = (float)xc;
+            D[k] = (float)(xc - (double)A[k]);
+            c[k] = D[k];
         }
-        gD = guard_offset(m, D);
-    };
-    /* time location of a phase: tc, tc + h/2, tc + h */
-    auto tloc_of = [&](int ph) {
-        const double tq = ph == PH_F0 ? is.tc : (ph == PH_K4 ? is.tc + is.h : is.tc + is.h / 2);
-        return (tq - f.tmin) * inv_span;
-    };
-    /* enter a probe phase: its walk starts at the probe's own element */
-    auto enter_probe = [&](int ph) {
-        phase = ph;
-        hops = 0;
-        const double tl = tloc_of(ph);
-        if (is.mp[ph].elem == -1) err = E_ELEM;
-        else if ((tl > 1 + TINY) || (tl < 0 - TINY)) err = E_TLOC;
-        else if (is.mp[ph].elem < 0 || is.mp[ph].elem >= m.ne) err = E_ELEM;
-        e = is.mp[ph].elem;
+        gc = guard_offset(m, c);
     };
     /* start of a step (the loop head of integration.c:344); false when the
      * interval is done or the step budget spent */
@@ -1207,34 +1289,46 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
             return false;
         }
         if ((is.tc + is.h - b) * (is.tc + is.h - a) > 0.0) is.h = sign_of(b - is.tc, b - a);
+        const double l0 = (is.tc - f.tmin) * inv_span, l1 = (is.tc + is.h - f.tmin) * inv_span;
+        tl0 = (float)l0;
+        tlh = (float)((is.tc + is.h / 2 - f.tmin) * inv_span); /* lies between l0 and l1 */
+        tl1 = (float)l1;
+        if ((l0 > 1 + TINY) || (l0 < 0 - TINY) || (l1 > 1 + TINY) || (l1 < 0 - TINY)) err = E_TLOC;
         return true;
     };
     anchor();
     float r = 0.f, s = 0.f, t = 0.f;
-    int ltie = 0; /* a locate-walk test hit d == -TINY */
-    if (!begin_step()) phase = PH_DONE;
-    else enter_probe(PH_F0);
-    if (err) phase = PH_DONE;
+    int e = q0, ftag = -1, vtag = -1;
+    int4 nd = make_int4(0, 0, 0, 0);
+    if (!begin_step() || err) phase = PH_DONE;
     while (phase != PH_DONE) {
-        /* ---- one containment test of this lane's walk (the element's
-         * connectivity is loaded beside its frame, for the velocity gather
-         * when the walk ends here) */
-        const int4 nd = ld32(m.conn, e);
-        const bool at_x = phase == PH_F0 || phase == PH_LOC;
+        /* ---- one containment test of this lane's walk */
+        if (e != ftag) {
+            nd = ld32(m.conn, e);
+            const Frame F = ld_frame<DIM>(m, e);
+            rows[0] = F.a0;
+            rows[64] = F.a1;
+            if (DIM == 3) rows[128] = F.a2;
+            rows[64 * (R::FRAME - 1)] = F.a3;
+            ftag = e;
+        }
         int slot = -1, dec;
         float ge;
-        nat_fast_c<DIM>(m, e, A, at_x ? D : dq, r, s, t, ge);
-        dec = decide_fast<DIM>(r, s, t, ge, at_x ? gD : gdq, slot);
+        {
+            Frame F;
+            F.a0 = rows[0];
+            F.a1 = rows[64];
+            F.a2 = DIM == 3 ? rows[128] : make_float4(0.f, 0.f, 0.f, 0.f);
+            F.a3 = rows[64 * (R::FRAME - 1)];
+            nat_frame<DIM>(F, A, c, r, s, t, ge);
+        }
+        dec = decide_fast<DIM>(r, s, t, ge, gc, slot);
         if (dec == 2) {
-            double x, y, z;
-            if (at_x) {
-                x = p.X[0];
-                y = p.X[1];
-                z = p.X[2];
-            } else {
-                x = (m.centre[0] + (double)A[0]) + (double)dq[0];
-                y = (m.centre[1] + (double)A[1]) + (double)dq[1];
-                z = (m.centre[2] + (double)A[2]) + (double)dq[2];
+            double x = p.X[0], y = p.X[1], z = p.X[2];
+            if (phase != PH_F0 && phase != PH_LOC) {
+                x = (m.centre[0] + (double)A[0]) + (double)c[0];
+                y = (m.centre[1] + (double)A[1]) + (double)c[1];
+                z = (m.centre[2] + (double)A[2]) + (double)c[2];
             }
             const ExactDec xd =
                 decide_exact_at<DIM>(m.X64, m.conn, e, x, y, z, phase == PH_LOC ? ACC_SEARCH : ACC_INTERP);
@@ -1243,7 +1337,7 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
             t = xd.t;
             slot = xd.slot;
             dec = xd.dec;
-            ltie |= xd.tie;
+            tie = tie || xd.tie;
         }
         if (dec < 0) {
             err = E_INDET;
@@ -1260,84 +1354,78 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
             }
         }
         /* ---- the walk ended: accepted at e, or left the mesh (e == -1) */
-        bool want = e >= 0;
-        double tl_i = 0.0;
+        const bool want = e >= 0;
+        hops = 0;
         if (phase == PH_LOC) {
-            p.elem = want ? e : -1;
-            /* a probe that left holds element -1 (and its left flag) */
-            const bool out = !want || is.mp[0].elem < 0 || is.mp[1].elem < 0 || is.mp[2].elem < 0 ||
-                             is.mp[3].elem < 0;
-            if (out) { /* exit: back to the step's start (integration.c:430-440) */
+            const int start = p.elem;
+            p.elem = e;
+            if (!want || gone) { /* exit: back to the step's start (integration.c:430-440) */
                 const double h6 = is.h * (1.0 / 6.0);
                 p.left = 1;
                 p.left_time = is.tc - is.h;
-                for (int c = 0; c < 3; c++) p.X[c] = p.X[c] - h6 * (double)S[c];
+                for (int k = 0; k < 3; k++) p.X[k] = p.X[k] - h6 * (double)S[k];
                 stop = p.left_time;
                 break;
             }
-            /* the next step; its first stage takes this element and these
+            if (!begin_step() || err) break;
+            phase = PH_F0;
+            /* the next step's first stage takes this element and these
              * coordinates when the locate started where the first stage
              * started and no test met the tie */
-            const bool reuse = !ltie && start == is.mp[0].elem;
-            if (!begin_step()) break;
-            if (!reuse) {
-                enter_probe(PH_F0);
-                if (err) break;
+            if (tie || start != q0) {
+                e = q0;
                 continue;
             }
-            tl_i = tloc_of(PH_F0);
-            if ((tl_i > 1 + TINY) || (tl_i < 0 - TINY)) {
-                err = E_TLOC;
-                break;
-            }
-            is.mp[0].elem = e;
-            phase = PH_F0;
-        } else {
-            if (want) is.mp[phase].elem = e;
-            else { /* the probe left: zero velocity for this stage (velocity.c:588-592) */
-                is.mp[phase].elem = -1;
-                is.mp[phase].left = 1;
-            }
-            tl_i = tloc_of(phase);
         }
-        /* ---- this stage's velocity and the next phase */
+        gone = gone || !want;
+        q0 = q1;
+        q1 = q2;
+        q2 = q3;
+        q3 = e;
+        /* ---- this stage's velocity (zero where the probe left, velocity.c:588-592) and the next phase */
         float k[3] = {0.f, 0.f, 0.f};
-        if (want) interp_nodes_f<MODE, DIM>(f, (float)tl_i, nd, r, s, t, k);
-        const float hf = (float)is.h, hh = 0.5f * hf;
-        if (phase == PH_F0) {
-            for (int c = 0; c < 3; c++) {
-                S[c] = k[c];
-                dq[c] = D[c] + hh * k[c];
+        if (want) {
+            NodeVel<MODE, DIM> g;
+            if (e != vtag) {
+                gather_vel<MODE, DIM>(f, nd, g);
+                vel_to_rows<MODE, DIM>(g, rows + 64 * R::FRAME);
+                vtag = e;
             }
-            gdq = guard_offset(m, dq);
-            enter_probe(PH_K2);
-        } else if (phase == PH_K2 || phase == PH_K3) {
-            const float w = phase == PH_K2 ? hh : hf;
-            for (int c = 0; c < 3; c++) {
-                S[c] = S[c] + 2.0f * k[c];
-                dq[c] = D[c] + w * k[c];
-            }
-            gdq = guard_offset(m, dq);
-            enter_probe(phase + 1);
-        } else { /* PH_K4: the step's increment, position and time */
+            vel_from_rows<MODE, DIM>(rows + 64 * R::FRAME, g);
+            interp_gathered<MODE, DIM>(f, g, phase == PH_F0 ? tl0 : phase == PH_K4 ? tl1 : tlh, r, s, t, k);
+        }
+        if (phase == PH_K4) { /* the step's increment, position and time */
             const double h = is.h, h6 = h * (1.0 / 6.0);
-            for (int c = 0; c < 3; c++) {
-                S[c] = S[c] + k[c];
-                p.X[c] = p.X[c] + h6 * (double)S[c];
+            for (int k3 = 0; k3 < 3; k3++) {
+                S[k3] = S[k3] + k[k3];
+                p.X[k3] = p.X[k3] + h6 * (double)S[k3];
             }
             is.tc = is.tc + h;
             if (!(fabs(h) <= hmin)) nsteps++;
             taken++;
             anchor();
-            phase = PH_LOC;
-            hops = 0;
-            ltie = 0;
-            start = p.elem;
+            tie = false;
             e = p.elem; /* a located element: the walks above keep p.elem >= 0 */
+        } else {
+            const float hf = (float)is.h, w = phase == PH_K3 ? hf : 0.5f * hf;
+            const bool first = phase == PH_F0;
+            for (int k3 = 0; k3 < 3; k3++) {
+                S[k3] = first ? k[k3] : S[k3] + 2.0f * k[k3];
+                c[k3] = D[k3] + w * k[k3];
+            }
+            gc = guard_offset(m, c);
+            e = q0;
         }
-        if (err) break;
+        phase++;
     }
     if (err) stop = b;
+    if (!ret) { /* suspended at a step's start */
+        is.mp[0].elem = q0;
+        is.mp[1].elem = q1;
+        is.mp[2].elem = q2;
+        is.mp[3].elem = q3;
+        for (int q = 0; q < 4; q++) is.mp[q].left = 0;
+    }
     return ret;
 }
 
@@ -1352,7 +1440,8 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
  *   (accumulation remainders) are Euler steps that keep the history. */
 template <int MODE, int DIM, int UNSTRUCT, int GEN>
 __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, IState &is, double a, double b, double dt,
-                            int itype_rt, int extrap, int max_steps, int &err, uint32_t &nsteps, double &stop) {
+                            int itype_rt, int extrap, int max_steps, int &err, uint32_t &nsteps, double &stop,
+                            float4 *rows = nullptr) {
 #pragma clang fp contract(off)
     /* GEN = 0 compiles RK4 only (no multistep state in registers) */
     const int itype = GEN ? itype_rt : INT_RK4;
@@ -1361,7 +1450,7 @@ __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, ISta
          * time; the GEN = 1 builds (other integrators, RK4 with extrapolation
          * or those integrals) keep the straight-line walks below and leave
          * the state machine's registers out */
-        if (!extrap) return rk4_sm<MODE, DIM>(m, f, p, is, a, b, dt, max_steps, err, nsteps, stop);
+        if (!extrap) return rk4_sm<MODE, DIM>(m, f, p, is, a, b, dt, max_steps, err, nsteps, stop, rows);
     }
     if (!is.started) {
         if (p.left) {
@@ -1690,7 +1779,7 @@ __device__ double rkf_run(const DevMesh &m, const DevField &f, PState &p, double
 /* Advect (ompVC/integration.c:22-45) over [t1, t2] in one go */
 template <int MODE, int DIM, int UNSTRUCT, int GEN = 1>
 __device__ __forceinline__ double advect(const DevMesh &m, const DevField &f, PState &p, double t1, double t2, int itype,
-                                         double dt, int extrap, int &err, uint32_t &nsteps) {
+                                         double dt, int extrap, int &err, uint32_t &nsteps, float4 *rows = nullptr) {
 #pragma clang fp contract(off)
     if (p.left && extrap) {
         for (int c = 0; c < 3; c++) p.X[c] = p.X[c] + p.V[c] * (t2 - t1);
@@ -1702,7 +1791,8 @@ __device__ __forceinline__ double advect(const DevMesh &m, const DevField &f, PS
     } else {
         IState is;
         is.started = 0;
-        interval_run<MODE, DIM, UNSTRUCT, GEN>(m, f, p, is, t1, t2, dt, itype, extrap, 0x7fffffff, err, nsteps, stop);
+        interval_run<MODE, DIM, UNSTRUCT, GEN>(m, f, p, is, t1, t2, dt, itype, extrap, 0x7fffffff, err, nsteps, stop,
+                                               rows);
     }
     if ((fabs(stop - t2) > TINY) && extrap)
         for (int c = 0; c < 3; c++) p.X[c] = p.X[c] + p.V[c] * (t2 - stop);

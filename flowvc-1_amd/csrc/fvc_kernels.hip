@@ -42,41 +42,38 @@ __device__ __forceinline__ int64_t xcd_block() {
     return x * per + (x < rem ? x : rem) + k;
 }
 
-__device__ inline void add_steps(unsigned long long *ctr, uint32_t ns) {
-    __shared__ unsigned int red[BLOCK / 64];
-    unsigned long long v = ns;
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) red[w] = (unsigned int)v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long s = 0;
-        for (int q = 0; q < (int)(blockDim.x >> 6); q++) s += red[q];
-        if (s) atomicAdd(ctr, s);
+/* The block's particle-steps into ctr[0] and, with IDLE, the number of its
+ * lanes whose particle was not integrated into ctr[1].  Each wave reports in
+ * the first of its own LDS rows, which it has finished with (the rows fill
+ * the block's share of the LDS), or in a small array where there are none. */
+template <int MODE, int DIM, int UNS, int GEN, bool IDLE>
+__device__ __forceinline__ void add_steps(unsigned long long *ctr, uint32_t ns, bool idle = false) {
+    constexpr int N = UNS && !GEN ? SmRows<MODE, DIM>::N : 0, W = N > 0 ? 256 * N : 2;
+    unsigned int *red;
+    if constexpr (N > 0) {
+        red = reinterpret_cast<unsigned int *>(sm_rows<MODE, DIM, UNS, GEN, BLOCK>() - threadIdx.x % 64) -
+              (threadIdx.x >> 6) * W;
+    } else {
+        __shared__ unsigned int s_red[2 * (BLOCK / 64)];
+        red = s_red;
     }
-}
-
-/* add_steps, plus the number of the block's lanes whose particle was not
- * integrated into ctr[1] */
-__device__ inline void add_steps_idle(unsigned long long *ctr, uint32_t ns, bool idle) {
-    __shared__ unsigned int red[BLOCK / 64], ired[BLOCK / 64];
-    unsigned long long v = ns;
+    unsigned int v = ns;
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    const unsigned int ni = (unsigned int)__popcll(__ballot(idle));
-    int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned int ni = IDLE ? (unsigned int)__popcll(__ballot(idle)) : 0;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (lane == 0) {
-        red[w] = (unsigned int)v;
-        ired[w] = ni;
+        red[w * W] = v;
+        red[w * W + 1] = ni;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long s = 0, si = 0;
         for (int q = 0; q < (int)(blockDim.x >> 6); q++) {
-            s += red[q];
-            si += ired[q];
+            s += red[q * W];
+            si += red[q * W + 1];
         }
         if (s) atomicAdd(ctr, s);
-        if (si) atomicAdd(ctr + 1, si);
+        if (IDLE && si) atomicAdd(ctr + 1, si);
     }
 }
 
@@ -143,14 +140,15 @@ __device__ __forceinline__ void advect_body(const DevMesh &m, const DevField &f,
             PState s;
             load_state(p, i, s, hist, extrap);
             int err = 0;
-            advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, extrap, err, ns);
+            advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, extrap, err, ns,
+                                        sm_rows<MODE, DIM, UNS, GEN, BLOCK>());
             if (err)
                 raise_err(eb, err, i);
             else
                 store_state(p, i, s, hist, extrap);
         }
     }
-    add_steps_idle(steps, ns, idle);
+    add_steps<MODE, DIM, UNS, GEN, true>(steps, ns, idle);
 }
 
 /* RK4 without extrapolation: no multistep state or particle velocity in
@@ -194,14 +192,15 @@ __device__ __forceinline__ void k_advect_times_body(const DevMesh &m, const DevF
             PState s;
             load_state(p, i, s, hist, extrap);
             int err = 0;
-            advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, extrap, err, ns);
+            advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, extrap, err, ns,
+                                        sm_rows<MODE, DIM, UNS, GEN, BLOCK>());
             if (err)
                 raise_err(eb, err, i);
             else
                 store_state(p, i, s, hist, extrap);
         }
     }
-    add_steps(steps, ns);
+    add_steps<MODE, DIM, UNS, GEN, false>(steps, ns);
 }
 
 template <int MODE, int DIM, int UNS>
@@ -1290,7 +1289,8 @@ __device__ __forceinline__ void ftle_advect_body(const DevMesh &m, const DevFiel
         PState s;
         load_state(d.p, i, s, false, extrap);
         int err = 0;
-        advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, extrap, err, ns);
+        advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, extrap, err, ns,
+                                    sm_rows<MODE, DIM, UNS, GEN, BLOCK>());
         if (err) raise_err(eb, err, i);
         d.advected[i] = 1;
         int ex = s.left && !extrap;
@@ -1303,7 +1303,7 @@ __device__ __forceinline__ void ftle_advect_body(const DevMesh &m, const DevFiel
         d.elem_new[i] = s.elem;
         if (extrap) d.p.left[i] = s.left;
     }
-    add_steps(steps, ns);
+    add_steps<MODE, DIM, UNS, GEN, false>(steps, ns);
 }
 
 template <int MODE, int DIM, int UNS>
@@ -1336,7 +1336,7 @@ __device__ void advect_copy(const DevMesh &m, const DevField &f, const FtleDev &
     s.elem = updated ? d.elem_new[idx] : d.p.elem[idx];
     s.left_time = 0.0;
     uint32_t ns = 0;
-    advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, 0, err, ns);
+    advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, 0, err, ns, sm_rows<MODE, DIM, UNS, GEN, BLOCK>());
 }
 
 /* Frame-start state of the stencils of one frame's triggered points, taken
@@ -1384,7 +1384,7 @@ __device__ void advect_snap(const DevMesh &m, const DevField &f, const EarlySnap
     s.elem = sn.elem[q * sn.cap + t];
     s.left_time = 0.0;
     uint32_t ns = 0;
-    advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, 0, err, ns);
+    advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, 0, err, ns, sm_rows<MODE, DIM, UNS, GEN, BLOCK>());
 }
 
 __device__ inline void ftle_value(double D[3][3], double dt_int, double &wt, double &wot, int &err, bool zero_time) {

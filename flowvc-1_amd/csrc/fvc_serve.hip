@@ -94,7 +94,7 @@ __device__ inline DevField srv_field(const SrvDev &S, int f) {
 }
 
 /* one particle for at most `budget` steps; returns the steps it took */
-template <int MODE, int GEN>
+template <int MODE, int GEN, int BS>
 __device__ uint32_t serve_particle(const DevMesh &m, const SrvDev &S, int i, int budget, int &r_out, int &fin) {
 #pragma clang fp contract(off)
     int fl = S.flags[i];
@@ -153,7 +153,8 @@ __device__ uint32_t serve_particle(const DevMesh &m, const SrvDev &S, int i, int
         const uint32_t before = ns;
         double stop;
         const int finished =
-            interval_run<MODE, 3, 1, GEN>(m, fld, s, is, ia, ib, S.dt, R.itype, 0, left_budget, err, ns, stop);
+            interval_run<MODE, 3, 1, GEN>(m, fld, s, is, ia, ib, S.dt, R.itype, 0, left_budget, err, ns, stop,
+                                        sm_rows<MODE, 3, 1, GEN, BS>());
         if (err) break;
         if (!finished) {
             fl |= SF_STARTED;
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(GEN ? 2 : FV
             const int idx = seg_lo + base + lane;
             int r = -1, fin = 0;
             uint32_t ns = 0;
-            if (idx < seg_hi) ns = serve_particle<MODE, GEN>(m, S, S.list_in[idx], budget, r, fin);
+            if (idx < seg_hi) ns = serve_particle<MODE, GEN, BS>(m, S, S.list_in[idx], budget, r, fin);
             total += ns;
             /* per-request step counts and phase counters: one atomic per wave
              * when the wave serves one request (the usual case: requests own

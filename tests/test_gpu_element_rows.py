@@ -1,0 +1,72 @@
+"""The RK4 state machine of the reduced-precision modes keeps each lane's
+element frame and node velocities in LDS rows.  Positions, exits and elements
+against the FP64 oracle at block and wave edges, with steps from a fraction of
+an element to several elements long, forward and backward."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+import cases
+from fvcpy import fvc, host
+
+sys.path.insert(0, os.path.join(cases.REPO, "oracle"))
+import oracle  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def _field(dims):
+    if dims == 3:
+        t = host.pipe(10, 10, 40, 1.0, 10.0)
+        xyz, conn, adj = host.tube_mesh(t)
+        sl = [host.tube_velocity(t, xyz, s * 0.02, 0.01, 77, s) for s in range(2)]
+        return [-1.0, 1.0, -1.0, 1.0, 0.0, 10.0], xyz, conn, adj, sl, lambda n: host.tube_seeds(t, n, 0.0, 10.0, 5)
+    xyz, conn, adj = cases.chan_mesh()
+    lo, hi = xyz.min(axis=0), xyz.max(axis=0)
+    sl = [np.stack([1.0 + np.sin(5 * xyz[:, 1] + s), 0.6 * np.cos(4 * xyz[:, 0] - s), 0 * xyz[:, 0]], axis=1) for s in range(2)]
+    rng = np.random.default_rng(6)
+    return ([lo[0], hi[0], lo[1], hi[1], 0.0, 0.0], xyz, conn, adj, sl, lambda n: rng.uniform(lo, hi, (n, 3)) * [1, 1, 0])
+
+
+# Position error against FP64 after time T: the stage velocities carry a
+# relative rounding of about 40 2^-24 in FP32 and of half an ulp of the
+# slice's largest value in 16 bits (2^-9, 2^-12), so |dx| <= rel umax T e^(G T)
+# with umax 3.3 and velocity gradients up to G = 4; an exit may differ only
+# for points that come that close to a wall.
+REL = {"f32": 40 * 2.0**-24, "bf16": 2.0**-9, "f16": 2.0**-12}
+
+
+@pytest.mark.parametrize("dims", [2, 3])
+@pytest.mark.parametrize("precision", ["f32", "bf16", "f16"])
+def test_rows_follow_the_oracle(dims, precision):
+    bounds, xyz, conn, adj, sl, seeds = _field(dims)
+    ctx = fvc.Context(dims, bounds, precision, 2, coords=xyz, conn=conn, adj=adj)
+    om = oracle.Mesh(dims, bounds, coords=xyz, conn=conn, adj=adj)
+    for s in range(2):
+        ctx.load_slice(s, 0.02 * s, sl[s])
+        om.set_slot(s, sl[s])
+    for n in (1, 63, 65, 257, 3000):
+        recs = ctx.seed_list(seeds(n))
+        for dt, t1, t2 in ((1e-3, 0.0, 0.02), (0.03, 0.0, 0.24), (7e-4, 0.02, 0.0)):
+            lo, hi = min(t1, t2), max(t1, t2)
+            om.set_interval(lo, hi)
+            ref = recs.copy()
+            assert om.advect(ref, t1, t2, dt) == 0
+            p = fvc.Particles(ctx, n)
+            p.set(recs)
+            print("rows dims %d %s n %d dt %g" % (dims, precision, n, dt), flush=True)
+            p.advect(t1, t2, 0, 1, lo, hi, dt)
+            got = p.get()
+            p.close()
+            stay = (got["LeftDomain"] == 0) & (ref["LeftDomain"] == 0)
+            tol = REL[precision] * 3.3 * (hi - lo) * np.exp(4 * (hi - lo))
+            assert np.abs(got["X"][stay] - ref["X"][stay]).max(initial=0.0) <= tol
+            differ = (got["LeftDomain"] != ref["LeftDomain"]).sum()
+            assert differ <= 1 + n * tol / 0.05
+            # the element held is the one that holds the position
+            at = np.ascontiguousarray(got["X"][got["LeftDomain"] == 0])
+            el = got["ElementIndex"][got["LeftDomain"] == 0]
+            np.testing.assert_array_equal(ctx.locate(at, el, fvc.LOCATE_WALK), el)
+    ctx.close()
