@@ -165,6 +165,7 @@ DevField bind_field(fvc_ctx *c, int lo, int hi, double tmin, double tmax) {
     f.scale_hi = c->slice_scale[hi];
     f.tmin = tmin;
     f.tmax = tmax;
+    f.vals = c->slice_vals[lo] | c->slice_vals[hi];
     return f;
 }
 
@@ -419,6 +420,7 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
     c->slices.assign(pp->max_slices, nullptr);
     c->slice_scale.assign(pp->max_slices, 1.0f);
     c->slice_time.assign(pp->max_slices, 0.0);
+    c->slice_vals.assign(pp->max_slices, VALS_INF | VALS_Z);
     c->sr_slices.assign(pp->max_slices, nullptr);
     memset(&c->mesh, 0, sizeof c->mesh);
     DevMesh &m = c->mesh;
@@ -481,6 +483,7 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
             m.cdel[2] = 0;
             m.cres[2] = 1;
         }
+        for (int a = 0; a < 3; a++) m.cinv[a] = fvc_near_inverse(m.cdel[a]);
         c->nvel = (int64_t)m.cres[0] * m.cres[1] * m.cres[2];
         /* strain-rate cells (strainrate.c:86-91): kmax = 1 in 2-D or for a single z layer */
         c->nsr = (int64_t)(m.cres[0] - 1) * (m.cres[1] - 1) * ((md->dims == 2 || m.cres[2] == 1) ? 1 : m.cres[2] - 1);
@@ -680,9 +683,16 @@ extern "C" int fvc_load_slice(fvc_ctx *c, int32_t slot, double timestamp, const 
     }
     std::vector<unsigned char> host(c->vel_stride * (size_t)n);
     float scale = 1.0f;
+    int vals = VALS_INF | VALS_Z;
     if (c->precision == FVC_PREC_F64) {
         double4 *h = (double4 *)host.data();
-        for (int64_t i = 0; i < n; i++) h[i] = make_double4(uvw[3 * i], uvw[3 * i + 1], uvw[3 * i + 2], 0.0);
+        bool inf = false, z = false;
+        for (int64_t i = 0; i < n; i++) {
+            h[i] = make_double4(uvw[3 * i], uvw[3 * i + 1], uvw[3 * i + 2], 0.0);
+            inf = inf | (fabs(h[i].x) == INFINITY) | (fabs(h[i].y) == INFINITY) | (fabs(h[i].z) == INFINITY);
+            z = z | (h[i].z != 0.0);
+        }
+        vals = (inf ? VALS_INF : 0) | (z ? VALS_Z : 0);
     } else if (c->precision == FVC_PREC_F32) {
         float4 *h = (float4 *)host.data();
         for (int64_t i = 0; i < n; i++)
@@ -703,6 +713,7 @@ extern "C" int fvc_load_slice(fvc_ctx *c, int32_t slot, double timestamp, const 
         hipStreamSynchronize(c->stream) != hipSuccess)
         return set_err(c, FVC_E_HIP, "slice upload");
     c->slice_scale[slot] = scale;
+    c->slice_vals[slot] = vals;
     c->slice_time[slot] = timestamp;
     return FVC_OK;
 }

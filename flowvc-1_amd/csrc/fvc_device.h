@@ -28,6 +28,7 @@
 
 #include <type_traits>
 
+#include "fvc_div.h"
 #include "fvc_root4.h"
 
 /* waves per SIMD the hot persistent and per-interval RK4 kernels are
@@ -52,6 +53,7 @@ struct DevMesh {
     double bounds[6];
     /* Cartesian velocity grid */
     double cmin[3], cdel[3];
+    double cinv[3]; /* 1 / cdel rounded to nearest, 0 where div_near does not apply */
     int cres[3];
     /* unstructured */
     const double4 *__restrict__ X64;
@@ -69,11 +71,15 @@ struct DevMesh {
     int hres[3];
 };
 
+enum { VALS_INF = 1, VALS_Z = 2 }; /* an infinity; a third component other than zero */
+
 /* Velocity slices bound for one interval: slot lo at tmin, hi at tmax. */
 struct DevField {
     const void *lo, *hi;
     float scale_lo, scale_hi;
     double tmin, tmax;
+    /* what the FP64 values of the two slices may hold (Cartesian meshes) */
+    int vals = VALS_INF | VALS_Z;
     /* strain-rate slices at tmin, tmax when the activation potential is integrated, else null */
     const double *sr_lo = nullptr, *sr_hi = nullptr;
     /* exposure time accumulators (per element: 128-bit fixed-point time, encounters), else null */
@@ -613,6 +619,11 @@ struct F3 {
     float x, y, z;
 };
 
+/* What a lane has stored in its LDS rows is read from there below this point
+ * also by the lanes that stored it: taken from their registers instead, the
+ * whole element would have to stay live beside the rows' copy. */
+__device__ __forceinline__ void reload_rows() { asm volatile("" ::: "memory"); }
+
 template <int MODE, int DIM>
 struct NodeVel {
     static constexpr int NN = DIM == 3 ? 4 : 3;
@@ -772,82 +783,257 @@ __device__ __forceinline__ int outside_domain(const DevMesh &m, double x, double
     return 0;
 }
 
-template <int DIM>
-__device__ __forceinline__ int outside_cart_vel(const DevMesh &m, const double X[3]) {
+/* (t - tmin) / (tmax - tmin), tinv = fvc_near_inverse(tmax - tmin) */
+__device__ __forceinline__ double time_loc(const DevField &f, double t, double tinv) {
 #pragma clang fp contract(off)
-    for (int a = 0; a < DIM; a++) {
-        double q = (X[a] - m.cmin[a]) / m.cdel[a];
-        int lo = (int)floor(q), hi = (int)ceil(q);
-        if (lo < 0 || hi > m.cres[a] - 1) return 1;
+    const double d = t - f.tmin, span = f.tmax - f.tmin;
+    return tinv != 0.0 ? fvc_div_near(d, span, tinv) : d / span;
+}
+
+/* x / 6 of the RK4 increment; infinities take the division.  The three
+ * quotients side by side: each is a chain of five dependent instructions. */
+__device__ __forceinline__ void sixths(double x[3]) {
+    if (fmax(fabs(x[0]), fmax(fabs(x[1]), fabs(x[2]))) < 1e300) {
+        for (int c = 0; c < 3; c++) x[c] = fvc_div_near(x[c], 6.0, 1.0 / 6.0);
+    } else {
+        for (int c = 0; c < 3; c++) x[c] = x[c] / 6;
     }
-    return 0;
+}
+
+/* Cell and local coordinates of X in the velocity grid, false outside it
+ * (velocity.c:257-457): q = (X - min) / del, outside where floor(q) < 0 or
+ * ceil(q) > res - 1, which for an integer bound is q < 0 or q > res - 1.
+ * The axes are computed side by side, without a branch between them. */
+template <int DIM>
+__device__ __forceinline__ bool cart_cell(const DevMesh &m, const double X[3], int cell[3], double loc[3]) {
+#pragma clang fp contract(off)
+    bool in = true, near = true;
+    double d[DIM], q[DIM], r[DIM];
+    for (int a = 0; a < DIM; a++) {
+        d[a] = X[a] - m.cmin[a];
+        near = near && m.cinv[a] != 0.0;
+    }
+    if (near)
+        for (int a = 0; a < DIM; a++) q[a] = fvc_div_near(d[a], m.cdel[a], m.cinv[a]);
+    else
+        for (int a = 0; a < DIM; a++) q[a] = d[a] / m.cdel[a];
+    for (int a = 0; a < DIM; a++) {
+        const double top = (double)(m.cres[a] - 1);
+        in = in && !(q[a] < 0.0) && !(q[a] > top) && !(fabs(d[a]) >= 1e280);
+        const double fl = floor(q[a]);
+        r[a] = d[a] - fl * m.cdel[a];
+        cell[a] = (int)fl;
+    }
+    if (near)
+        for (int a = 0; a < DIM; a++) r[a] = fvc_div_near(r[a], m.cdel[a], m.cinv[a]);
+    else
+        for (int a = 0; a < DIM; a++) r[a] = r[a] / m.cdel[a];
+    for (int a = 0; a < DIM; a++) { /* the last node belongs to the last cell */
+        const bool end = cell[a] == m.cres[a] - 1;
+        loc[a] = end ? 1.0 : r[a];
+        cell[a] = end ? cell[a] - 1 : cell[a];
+    }
+    return in;
+}
+
+/* The corners of a cell, (x, y, z) offsets in the bits (4, 2, 1) of the
+ * corner number; a 2-D cell's are 0, 2, 4 and 6. */
+template <int MODE, int DIM>
+struct CartCorners {
+    static constexpr int NQ = 1 << DIM, STEP = DIM == 3 ? 1 : 2;
+    static constexpr int STRIDE = MODE == P_F64 ? 32 : MODE == P_F32 ? 16 : 8;
+    const char *row[4]; /* corners (0, y, z), index 2 y + z; corner x + 1 follows at STRIDE */
+    __device__ __forceinline__ void at(const DevMesh &m, const void *base, int64_t c0) {
+        const int64_t nx = m.cres[0] * (int64_t)STRIDE;
+        row[0] = (const char *)base + c0 * STRIDE;
+        row[2] = row[0] + nx;
+        if (DIM == 3) {
+            row[1] = row[0] + nx * m.cres[1];
+            row[3] = row[1] + nx;
+        }
+    }
+    __device__ __forceinline__ const char *corner(int q) const { return row[q & 3] + (q >> 2) * STRIDE; }
+};
+
+template <int DIM>
+__device__ __forceinline__ int64_t cart_index(const DevMesh &m, const int cell[3]) {
+    const int64_t row = DIM == 3 ? (int64_t)cell[2] * m.cres[1] + cell[1] : (int64_t)cell[1];
+    return row * m.cres[0] + cell[0];
+}
+
+/* LDS rows of the Cartesian RK4 kernels: the corner velocities of the cell a
+ * lane interpolated in last (both slices), as SmRows holds an element's.  A
+ * stage moves a fraction of a cell, so gathering only after a change of cell
+ * cuts the gathers several times over.  In FP64 only in 2-D, for slices whose
+ * third component is zero: a 3-D cell is 384 bytes, which would leave 6 waves
+ * on a CU.  300,007 points in random order on an 80x64x48 grid, FP32, 20
+ * steps: 2,244 us, bound by the lines those gathers pull through the L2, to
+ * 265 us. */
+template <int MODE, int DIM>
+struct CartRows {
+    static constexpr int NQ = 1 << DIM, W = MODE == P_F64 ? 4 : MODE == P_F32 ? DIM : 2;
+    static constexpr int N = MODE == P_F64 && DIM == 3 ? 0 : (2 * NQ * W + 3) / 4;
+};
+
+/* this lane's last cell and its rows (rows null: gather every time) */
+struct CartLast {
+    float4 *rows = nullptr;
+    int64_t cell = -1;
+};
+
+template <int DIM>
+__device__ __forceinline__ void cart_velocity_f64(const DevMesh &m, const DevField &f, double tl, const int cell[3],
+                                                  const double loc[3], CartLast &last, double out[3]) {
+#pragma clang fp contract(off)
+    using C = CartCorners<P_F64, DIM>;
+    const int64_t c0 = cart_index<DIM>(m, cell);
+    const double tw[2] = {1 - tl, tl};
+    /* a corner's weight: products left to right, time, x, y, z */
+    auto weight = [&](int s, int q) {
+        double w = tw[s] * ((q & 4) ? loc[0] : (1 - loc[0])) * ((q & 2) ? loc[1] : (1 - loc[1]));
+        if (DIM == 3) w = w * ((q & 1) ? loc[2] : (1 - loc[2]));
+        return w;
+    };
+    double acc[3] = {0.0, 0.0, 0.0};
+    if (DIM == 2 && !f.vals && last.rows) { /* finite, third component zero */
+        if (c0 != last.cell) {
+            C cc[2];
+            cc[0].at(m, f.lo, c0);
+            cc[1].at(m, f.hi, c0);
+            for (int k = 0; k < 8; k++)
+                last.rows[64 * k] = *reinterpret_cast<const float4 *>(cc[k >> 2].corner((k & 3) * 2));
+            last.cell = c0;
+        }
+        reload_rows();
+        for (int s = 0; s < 2; s++)
+            for (int k = 0; k < 4; k++) {
+                const double2 v = *reinterpret_cast<const double2 *>(last.rows + 64 * (4 * s + k));
+                const double w = weight(s, 2 * k);
+                acc[0] = s == 0 && k == 0 ? v.x * w : acc[0] + v.x * w;
+                acc[1] = s == 0 && k == 0 ? v.y * w : acc[1] + v.y * w;
+            }
+        for (int c = 0; c < 3; c++) out[c] = acc[c];
+        return;
+    }
+    double big[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1 /* both slices' corners at once spill */
+    for (int s = 0; s < 2; s++) {
+        C cc;
+        cc.at(m, s ? f.hi : f.lo, c0);
+        double v[8][3];
+        for (int q = 0; q < 8; q += C::STEP) {
+            const double *p = reinterpret_cast<const double *>(cc.corner(q));
+            for (int c = 0; c < 3; c++) v[q][c] = p[c];
+        }
+        for (int q = 0; q < 8; q += C::STEP) {
+            const double w = weight(s, q);
+            for (int c = 0; c < 3; c++) acc[c] = s == 0 && q == 0 ? v[q][c] * w : acc[c] + v[q][c] * w;
+        }
+        /* In 2-D the reference's formula also adds every corner of the plane
+         * k + 1, the same node, with weight zero: nothing, unless the node
+         * holds an infinity. */
+        if (DIM == 2 && (f.vals & VALS_INF))
+            for (int q = 0; q < 8; q += C::STEP)
+                for (int c = 0; c < 3; c++) big[c] = fmax(big[c], fabs(v[q][c]));
+    }
+    if (DIM == 2 && (f.vals & VALS_INF))
+        for (int c = 0; c < 3; c++) acc[c] = acc[c] + big[c] * 0.0;
+    for (int c = 0; c < 3; c++) out[c] = acc[c];
+}
+
+/* one corner's words as loaded: FP32 components, or four 16-bit values */
+template <int MODE, int DIM>
+__device__ __forceinline__ void cart_words(const char *p, float *w) {
+    if constexpr (MODE == P_F32) {
+        const float4 v = *reinterpret_cast<const float4 *>(p);
+        w[0] = v.x;
+        w[1] = v.y;
+        if (DIM == 3) w[2] = v.z;
+    } else {
+        const uint2 v = *reinterpret_cast<const uint2 *>(p);
+        w[0] = __uint_as_float(v.x);
+        w[1] = __uint_as_float(v.y);
+    }
 }
 
 template <int MODE, int DIM>
-__device__ __forceinline__ void vel_cart(const DevMesh &m, const DevField &f, double tloc, const double X[3], int &left,
-                                         double out[3]) {
-#pragma clang fp contract(off)
-    if (outside_cart_vel<DIM>(m, X)) {
-        out[0] = out[1] = out[2] = 0.0;
-        left = 1;
-        return;
-    }
-    int cell[3] = {0, 0, 0};
-    double loc[3] = {0.0, 0.0, 0.0};
-    for (int a = 0; a < DIM; a++) {
-        cell[a] = (int)floor((X[a] - m.cmin[a]) / m.cdel[a]);
-        if (cell[a] == m.cres[a] - 1) {
-            cell[a] = m.cres[a] - 2;
-            loc[a] = 1.0;
-        } else {
-            loc[a] = (X[a] - m.cmin[a] - cell[a] * m.cdel[a]) / m.cdel[a];
-        }
-    }
-    const int64_t nx = m.cres[0], ny = m.cres[1];
-    const int i = cell[0], j = cell[1], k = cell[2], k1 = DIM == 3 ? k + 1 : k;
-    int64_t c[8] = {((int64_t)k * ny + j) * nx + i,           ((int64_t)k1 * ny + j) * nx + i,
-                    ((int64_t)k * ny + j + 1) * nx + i,       ((int64_t)k1 * ny + j + 1) * nx + i,
-                    ((int64_t)k * ny + j) * nx + i + 1,       ((int64_t)k1 * ny + j) * nx + i + 1,
-                    ((int64_t)k * ny + j + 1) * nx + i + 1,   ((int64_t)k1 * ny + j + 1) * nx + i + 1};
-    if constexpr (MODE == P_F64) {
-        double tl = tloc, xl = loc[0], yl = loc[1], zl = loc[2];
-        /* weights w[slot][corner], corner bits (x,y,z) = (4,2,1); products left to right */
-        double w0[8], w1[8];
-        for (int q = 0; q < 8; q++) {
-            double wx = (q & 4) ? xl : (1 - xl), wy = (q & 2) ? yl : (1 - yl), wz = (q & 1) ? zl : (1 - zl);
-            w1[q] = (tl) * wx * wy * wz;
-            w0[q] = (1 - tl) * wx * wy * wz;
-        }
-        double A[8][3], B[8][3];
-        for (int q = 0; q < 8; q++) {
-            load_vel<MODE>(f.lo, 1.0f, c[q], A[q]);
-            load_vel<MODE>(f.hi, 1.0f, c[q], B[q]);
-        }
-        for (int cc = 0; cc < 3; cc++) {
-            double acc = A[0][cc] * w0[0];
-            for (int q = 1; q < 8; q++) acc = acc + A[q][cc] * w0[q];
-            for (int q = 0; q < 8; q++) acc = acc + B[q][cc] * w1[q];
-            out[cc] = acc;
-        }
+__device__ __forceinline__ void cart_value(const float *w, float scale, float v[3]) {
+    if constexpr (MODE == P_F32) {
+        v[0] = w[0];
+        v[1] = w[1];
+        v[2] = DIM == 3 ? w[2] : 0.0f;
     } else {
-        using VT = typename VelT<MODE>::T;
-        float tl = (float)tloc, xl = (float)loc[0], yl = (float)loc[1], zl = (float)loc[2];
-        float acc[3] = {0.f, 0.f, 0.f};
-        const int nq = DIM == 3 ? 8 : 8;
-        for (int q = 0; q < nq; q++) {
-            if (DIM == 2 && (q & 1)) continue; /* 2-D: the k+1 plane repeats k with zero weight */
-            float wx = (q & 4) ? xl : (1.f - xl), wy = (q & 2) ? yl : (1.f - yl);
-            float wz = DIM == 3 ? ((q & 1) ? zl : (1.f - zl)) : 1.f;
-            float w = wx * wy * wz;
-            VT a[3], b[3];
-            load_vel<MODE>(f.lo, f.scale_lo, c[q], a);
-            load_vel<MODE>(f.hi, f.scale_hi, c[q], b);
-            for (int cc = 0; cc < 3; cc++) acc[cc] += w * (a[cc] + tl * (b[cc] - a[cc]));
-        }
-        out[0] = acc[0];
-        out[1] = acc[1];
-        out[2] = DIM == 3 ? (double)acc[2] : 0.0;
+        node_comp<MODE>(make_uint2(__float_as_uint(w[0]), __float_as_uint(w[1])), v);
+        for (int c = 0; c < 3; c++) v[c] = v[c] * scale;
     }
+}
+
+template <int MODE, int DIM>
+__device__ __forceinline__ void cart_interp_f32(const DevField &f, const float *w, double tloc, const double loc[3],
+                                                double out[3]) {
+#pragma clang fp contract(off)
+    using C = CartCorners<MODE, DIM>;
+    using R = CartRows<MODE, DIM>;
+    const float tl = (float)tloc, xl = (float)loc[0], yl = (float)loc[1], zl = (float)loc[2];
+    float acc[3] = {0.f, 0.f, 0.f};
+    for (int k = 0; k < R::NQ; k++) {
+        const int q = k * C::STEP;
+        const float wx = (q & 4) ? xl : (1.f - xl), wy = (q & 2) ? yl : (1.f - yl);
+        float g = wx * wy;
+        if (DIM == 3) g = g * ((q & 1) ? zl : (1.f - zl));
+        float a[3], b[3];
+        cart_value<MODE, DIM>(w + 2 * R::W * k, f.scale_lo, a);
+        cart_value<MODE, DIM>(w + 2 * R::W * k + R::W, f.scale_hi, b);
+        for (int c = 0; c < 3; c++) acc[c] += g * (a[c] + tl * (b[c] - a[c]));
+    }
+    out[0] = acc[0];
+    out[1] = acc[1];
+    out[2] = DIM == 3 ? (double)acc[2] : 0.0;
+}
+
+template <int MODE, int DIM>
+__device__ __forceinline__ void cart_velocity_f32(const DevMesh &m, const DevField &f, double tloc, const int cell[3],
+                                                  const double loc[3], CartLast &last, double out[3]) {
+#pragma clang fp contract(off)
+    using C = CartCorners<MODE, DIM>;
+    using R = CartRows<MODE, DIM>;
+    const int64_t c0 = cart_index<DIM>(m, cell);
+    /* corner by corner: the lo slice's words, then the hi slice's */
+    if (!last.rows || c0 != last.cell) {
+        float w[4 * R::N];
+        C lo, hi;
+        lo.at(m, f.lo, c0);
+        hi.at(m, f.hi, c0);
+        for (int q = 0; q < R::NQ; q++) {
+            cart_words<MODE, DIM>(lo.corner(q * C::STEP), w + 2 * R::W * q);
+            cart_words<MODE, DIM>(hi.corner(q * C::STEP), w + 2 * R::W * q + R::W);
+        }
+        if (!last.rows) {
+            cart_interp_f32<MODE, DIM>(f, w, tloc, loc, out);
+            return;
+        }
+        for (int k = 0; k < R::N; k++)
+            last.rows[64 * k] = make_float4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+        last.cell = c0;
+    }
+    reload_rows();
+    float w[4 * R::N];
+    for (int k = 0; k < R::N; k++) {
+        const float4 v = last.rows[64 * k];
+        w[4 * k] = v.x;
+        w[4 * k + 1] = v.y;
+        w[4 * k + 2] = v.z;
+        w[4 * k + 3] = v.w;
+    }
+    cart_interp_f32<MODE, DIM>(f, w, tloc, loc, out);
+}
+
+/* velocity at a position inside the velocity grid */
+template <int MODE, int DIM>
+__device__ __forceinline__ void cart_velocity(const DevMesh &m, const DevField &f, double tloc, const int cell[3],
+                                              const double loc[3], CartLast &last, double out[3]) {
+    if constexpr (MODE == P_F64) cart_velocity_f64<DIM>(m, f, tloc, cell, loc, last, out);
+    else cart_velocity_f32<MODE, DIM>(m, f, tloc, cell, loc, last, out);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -887,8 +1073,9 @@ __device__ __forceinline__ void get_velocity(const DevMesh &m, const DevField &f
         p.elem = pr.elem;
         p.left = pr.left;
     } else {
-        int lft = 0;
-        if (outside_cart_vel<DIM>(m, p.X)) {
+        int cell[3];
+        double loc[3];
+        if (!cart_cell<DIM>(m, p.X, cell, loc)) {
             out[0] = out[1] = out[2] = 0.0;
             p.left = 1;
             return;
@@ -897,17 +1084,17 @@ __device__ __forceinline__ void get_velocity(const DevMesh &m, const DevField &f
             err = E_TLOC;
             return;
         }
-        vel_cart<MODE, DIM>(m, f, tloc, p.X, lft, out);
-        if (lft) p.left = 1;
+        CartLast none;
+        cart_velocity<MODE, DIM>(m, f, tloc, cell, loc, none, out);
     }
 }
 
 /* velocity at a probe position for a stage (probe owns its element / flag) */
 template <int MODE, int DIM, int UNSTRUCT>
 __device__ __forceinline__ void stage_velocity(const DevMesh &m, const DevField &f, double tq, const double X[3],
-                                               Probe &pr, double out[3], int &err) {
+                                               Probe &pr, double out[3], int &err, double tinv, CartLast &last) {
 #pragma clang fp contract(off)
-    double tloc = (tq - f.tmin) / (f.tmax - f.tmin);
+    const double tloc = time_loc(f, tq, tinv);
     if (UNSTRUCT) {
         if (pr.elem == -1) {
             err = E_ELEM;
@@ -919,7 +1106,9 @@ __device__ __forceinline__ void stage_velocity(const DevMesh &m, const DevField 
         }
         vel_unstruct<MODE, DIM>(m, f, tloc, X[0], X[1], X[2], pr, out, err);
     } else {
-        if (outside_cart_vel<DIM>(m, X)) {
+        int cell[3];
+        double loc[3];
+        if (!cart_cell<DIM>(m, X, cell, loc)) {
             out[0] = out[1] = out[2] = 0.0;
             pr.left = 1;
             return;
@@ -928,9 +1117,7 @@ __device__ __forceinline__ void stage_velocity(const DevMesh &m, const DevField 
             err = E_TLOC;
             return;
         }
-        int lft = 0;
-        vel_cart<MODE, DIM>(m, f, tloc, X, lft, out);
-        if (lft) pr.left = 1;
+        cart_velocity<MODE, DIM>(m, f, tloc, cell, loc, last, out);
     }
 }
 
@@ -1171,11 +1358,16 @@ struct SmRows {
     static constexpr int N = MODE == P_F64 ? 0 : FRAME + VEL;
 };
 
-/* this lane's rows in a block of BS lanes (null in the kernels that do not
- * run the state machine) */
+/* rows per lane of the RK4 kernels (GEN = 0), and this lane's in a block of
+ * BS lanes (null where there are none) */
+template <int MODE, int DIM, int UNS, int GEN>
+constexpr int lane_rows() {
+    return GEN ? 0 : UNS ? SmRows<MODE, DIM>::N : CartRows<MODE, DIM>::N;
+}
+
 template <int MODE, int DIM, int UNS, int GEN, int BS>
 __device__ __forceinline__ float4 *sm_rows() {
-    constexpr int N = UNS && !GEN ? SmRows<MODE, DIM>::N : 0;
+    constexpr int N = lane_rows<MODE, DIM, UNS, GEN>();
     if constexpr (N > 0) {
         __shared__ float4 s_rows[N * BS];
         return s_rows + (threadIdx.x >> 6) * (64 * N) + (threadIdx.x & 63);
@@ -1312,6 +1504,7 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
             rows[64 * (R::FRAME - 1)] = F.a3;
             ftag = e;
         }
+        reload_rows();
         int slot = -1, dec;
         float ge;
         {
@@ -1391,6 +1584,7 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
                 vel_to_rows<MODE, DIM>(g, rows + 64 * R::FRAME);
                 vtag = e;
             }
+            reload_rows();
             vel_from_rows<MODE, DIM>(rows + 64 * R::FRAME, g);
             interp_gathered<MODE, DIM>(f, g, phase == PH_F0 ? tl0 : phase == PH_K4 ? tl1 : tlh, r, s, t, k);
         }
@@ -1429,6 +1623,81 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
     return ret;
 }
 
+/* RK4 on a Cartesian grid (integration.c:317-462) without strain rate or
+ * extrapolation.  One copy of the stage's interpolation in a loop over the
+ * four stages, with the weighted slope sum built as they come, in the
+ * reference's order: four copies side by side hold all four slopes and spill
+ * (the FP64 3-D kernel 80 registers).  What bounds the FP64 kernel is its
+ * chain of dependent instructions: about 180 a stage, 490 with the divisions
+ * and the zero-weight corners.  512x256 FTLE points of the double gyre, 50
+ * steps: 499 us; without those divisions and corners 264 us; with the axes'
+ * quotients side by side and the cell's corners in LDS 209 us. */
+template <int MODE, int DIM>
+__device__ int rk4_cart(const DevMesh &m, const DevField &f, PState &p, IState &is, double a, double b, double dt,
+                        int max_steps, int &err, uint32_t &nsteps, double &stop, float4 *rows) {
+#pragma clang fp contract(off)
+    if (!is.started) {
+        if (p.left) {
+            err = E_LEFT;
+            stop = b;
+            return 1;
+        }
+        is.tc = a;
+        is.h = sign_of(dt, b - a);
+        is.started = 1;
+    }
+    const double hmin = 1e-12 * fabs(dt), tinv = fvc_near_inverse(f.tmax - f.tmin);
+    CartLast last;
+    last.rows = rows;
+    int taken = 0;
+    stop = b;
+    while ((is.tc - b) * (b - a) < 0.0) {
+        if (taken == max_steps) return 0;
+        if ((is.tc + is.h - b) * (is.tc + is.h - a) > 0.0) is.h = sign_of(b - is.tc, b - a);
+        const double h = is.h;
+        double Y[3], S[3] = {0.0, 0.0, 0.0};
+        bool out = false;
+        for (int c = 0; c < 3; c++) Y[c] = p.X[c];
+#pragma unroll 1
+        for (int stage = 0; stage < 4; stage++) {
+            const double tq = stage == 0 ? is.tc : stage == 3 ? is.tc + h : is.tc + h / 2;
+            double k[3] = {0.0, 0.0, 0.0}, loc[3];
+            int cell[3];
+            if (cart_cell<DIM>(m, Y, cell, loc)) {
+                const double tloc = time_loc(f, tq, tinv);
+                if ((tloc > 1 + TINY) || (tloc < 0 - TINY)) {
+                    err = E_TLOC;
+                    break;
+                }
+                cart_velocity<MODE, DIM>(m, f, tloc, cell, loc, last, k);
+            } else {
+                out = true; /* zero velocity for this stage */
+            }
+            const double w = stage == 2 ? 1.0 : 0.5, u = stage == 3 ? 1.0 : 2.0;
+            for (int c = 0; c < 3; c++) {
+                S[c] = stage == 0 ? k[c] : S[c] + u * k[c];
+                Y[c] = p.X[c] + w * k[c] * h;
+            }
+        }
+        if (err) return 1;
+        double inc[3];
+        for (int c = 0; c < 3; c++) inc[c] = h * S[c];
+        sixths(inc);
+        for (int c = 0; c < 3; c++) p.X[c] = p.X[c] + inc[c];
+        is.tc = is.tc + h;
+        if (!(fabs(h) <= hmin)) nsteps++;
+        taken++;
+        if (out || outside_domain(m, p.X[0], p.X[1], p.X[2])) {
+            p.left = 1;
+            p.left_time = is.tc - h;
+            for (int c = 0; c < 3; c++) p.X[c] = p.X[c] - inc[c];
+            stop = p.left_time;
+            return 1;
+        }
+    }
+    return 1;
+}
+
 /* Returns 1 when the interval is finished (end reached, point exited or an
  * error), with *stop the stop time; 0 when max_steps were taken first.
  *   RK4   ompVC/integration.c:317-462
@@ -1451,6 +1720,9 @@ __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, ISta
          * or those integrals) keep the straight-line walks below and leave
          * the state machine's registers out */
         if (!extrap) return rk4_sm<MODE, DIM>(m, f, p, is, a, b, dt, max_steps, err, nsteps, stop, rows);
+    }
+    if constexpr (!UNSTRUCT && !GEN) {
+        if (!extrap) return rk4_cart<MODE, DIM>(m, f, p, is, a, b, dt, max_steps, err, nsteps, stop, rows);
     }
     if (!is.started) {
         if (p.left) {
@@ -1499,6 +1771,9 @@ __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, ISta
     using KT = typename std::conditional<FAST, float, double>::type;
     /* FAST: time locations as (t - tmin) times one reciprocal of the frame span */
     const double inv_span = FAST ? 1.0 / (f.tmax - f.tmin) : 0.0;
+    const double tinv = FAST ? 0.0 : fvc_near_inverse(f.tmax - f.tmin);
+    CartLast last;
+    if (!UNSTRUCT && !GEN) last.rows = rows;
     while ((is.tc - b) * (b - a) < 0.0) {
         if (taken == max_steps) return 0;
         if ((is.tc + is.h - b) * (is.tc + is.h - a) > 0.0) is.h = sign_of(b - is.tc, b - a);
@@ -1518,7 +1793,7 @@ __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, ISta
             for (int c = 0; c < 3; c++) inc[c] = h * ve[c];
         } else {
             if (UNSTRUCT && c_elem >= 0) {
-                const double tloc = FAST ? (tc - f.tmin) * inv_span : (tc - f.tmin) / (f.tmax - f.tmin);
+                const double tloc = FAST ? (tc - f.tmin) * inv_span : time_loc(f, tc, tinv);
                 if ((tloc > 1 + TINY) || (tloc < 0 - TINY)) {
                     err = E_TLOC;
                     break;
@@ -1528,7 +1803,7 @@ __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, ISta
                 else interp_unstruct<MODE, DIM>(m, f, tloc, c_elem, c_r, c_s, c_t, f0);
             } else {
                 if constexpr (FAST) stage_velocity_x<MODE, DIM>(m, f, (tc - f.tmin) * inv_span, p.X, is.mp[0], f0, err);
-                else stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc, p.X, is.mp[0], f0, err);
+                else stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc, p.X, is.mp[0], f0, err, tinv, last);
             }
             c_elem = -1;
             if (err) break;
@@ -1574,15 +1849,16 @@ __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, ISta
             } else {
                 double k2[3], k3[3], k4[3], Y[3];
                 for (int c = 0; c < 3; c++) Y[c] = p.X[c] + 0.5 * f0[c] * h;
-                stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + h / 2, Y, is.mp[1], k2, err);
+                stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + h / 2, Y, is.mp[1], k2, err, tinv, last);
                 if (err) break;
                 for (int c = 0; c < 3; c++) Y[c] = p.X[c] + 0.5 * k2[c] * h;
-                stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + h / 2, Y, is.mp[2], k3, err);
+                stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + h / 2, Y, is.mp[2], k3, err, tinv, last);
                 if (err) break;
                 for (int c = 0; c < 3; c++) Y[c] = p.X[c] + k3[c] * h;
-                stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + h, Y, is.mp[3], k4, err);
+                stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + h, Y, is.mp[3], k4, err, tinv, last);
                 if (err) break;
-                for (int c = 0; c < 3; c++) inc[c] = h * (f0[c] + 2 * k2[c] + 2 * k3[c] + k4[c]) / 6;
+                for (int c = 0; c < 3; c++) inc[c] = h * (f0[c] + 2 * k2[c] + 2 * k3[c] + k4[c]);
+                sixths(inc);
             }
             (void)ab_step;
         }
@@ -1685,6 +1961,8 @@ __device__ double rkf_run(const DevMesh &m, const DevField &f, PState &p, double
     const double hmax = f.rkf_max, hmin = f.rkf_min, tol = f.rkf_tol;
     const bool ap = f.sr_lo != nullptr;                 /* activation potential (integration.c:534-539, 671-677) */
     const bool cet = UNSTRUCT && f.cet_lo != nullptr;   /* exposure time (integration.c:650-670) */
+    const double tinv = fvc_near_inverse(f.tmax - f.tmin);
+    CartLast last; /* gathers every time */
     double h = sign_of(hmax, b - a), tc = a;
     double k1[3], k2[3], k3[3], k4[3], k5[3], k6[3], Y[3];
     while ((tc - b) * (b - a) < 0.0) {
@@ -1694,23 +1972,23 @@ __device__ double rkf_run(const DevMesh &m, const DevField &f, PState &p, double
             sr0 = strain_rate<DIM, UNSTRUCT>(m, f, tc, p, err);
             if (err) return b;
         }
-        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc, p.X, mp[0], k1, err);
+        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc, p.X, mp[0], k1, err, tinv, last);
         if (err) return b;
         for (int c = 0; c < 3; c++) Y[c] = p.X[c] + 0.25 * k1[c] * h;
-        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + 0.25 * h, Y, mp[1], k2, err);
+        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + 0.25 * h, Y, mp[1], k2, err, tinv, last);
         if (err) return b;
         for (int c = 0; c < 3; c++) Y[c] = p.X[c] + (a3 * k1[c] + b3 * k2[c]) * h;
-        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + 0.375 * h, Y, mp[2], k3, err);
+        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + 0.375 * h, Y, mp[2], k3, err, tinv, last);
         if (err) return b;
         for (int c = 0; c < 3; c++) Y[c] = p.X[c] + (a4 * k1[c] + b4 * k2[c] + c4 * k3[c]) * h;
-        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + (12.0 * h) / 13.0, Y, mp[3], k4, err);
+        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + (12.0 * h) / 13.0, Y, mp[3], k4, err, tinv, last);
         if (err) return b;
         for (int c = 0; c < 3; c++) Y[c] = p.X[c] + (a5 * k1[c] + b5 * k2[c] + c5 * k3[c] + d5 * k4[c]) * h;
-        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + h, Y, mp[4], k5, err);
+        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + h, Y, mp[4], k5, err, tinv, last);
         if (err) return b;
         for (int c = 0; c < 3; c++)
             Y[c] = p.X[c] + (a6 * k1[c] + b6 * k2[c] + c6 * k3[c] + d6 * k4[c] + e6 * k5[c]) * h;
-        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + 0.5 * h, Y, mp[5], k6, err);
+        stage_velocity<MODE, DIM, UNSTRUCT>(m, f, tc + 0.5 * h, Y, mp[5], k6, err, tinv, last);
         if (err) return b;
         if (mp[0].left || mp[1].left || mp[2].left || mp[3].left || mp[4].left || mp[5].left) {
             p.left = 1;

@@ -37,6 +37,7 @@ struct fvc_ctx {
     std::vector<void *> slices;
     std::vector<float> slice_scale;
     std::vector<double> slice_time;
+    std::vector<int> slice_vals; /* Cartesian meshes: VALS_* of each slice */
     int64_t nvel;       /* nodes per slice */
     size_t vel_stride;  /* bytes per node */
     /* resident strain-rate slices (activation potential), FP64, one per slot */

@@ -48,7 +48,7 @@ __device__ __forceinline__ int64_t xcd_block() {
  * the block's share of the LDS), or in a small array where there are none. */
 template <int MODE, int DIM, int UNS, int GEN, bool IDLE>
 __device__ __forceinline__ void add_steps(unsigned long long *ctr, uint32_t ns, bool idle = false) {
-    constexpr int N = UNS && !GEN ? SmRows<MODE, DIM>::N : 0, W = N > 0 ? 256 * N : 2;
+    constexpr int N = lane_rows<MODE, DIM, UNS, GEN>(), W = N > 0 ? 256 * N : 2;
     unsigned int *red;
     if constexpr (N > 0) {
         red = reinterpret_cast<unsigned int *>(sm_rows<MODE, DIM, UNS, GEN, BLOCK>() - threadIdx.x % 64) -
@@ -156,9 +156,7 @@ __device__ __forceinline__ void advect_body(const DevMesh &m, const DevField &f,
  * The reduced-precision state machine on unstructured meshes fits 4
  * waves/SIMD (at most 128 VGPRs) without spills; the FP64 and Cartesian
  * builds are held to 3 (168), which hides more of the gather latency than
- * their natural allocation.  The 3-D FP64 Cartesian build spills about 80
- * VGPRs at 3 waves and still runs 16% faster than at 2 waves without spills
- * (2M particles on a 128^3 grid: 0.283 s against 0.336 s). */
+ * their natural allocation. */
 #define FVC_RK4_WAVES(MODE, UNS) ((MODE) != P_F64 && (UNS) ? 4 : FVC_HOT_WAVES)
 template <int MODE, int DIM, int UNS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_RK4_WAVES(MODE, UNS)))) void k_advect(
@@ -168,9 +166,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_RK4_W
     advect_body<MODE, DIM, UNS, 0>(m, f, p, index, begin, count, t1, t2, itype, dt, 0, eb, steps);
 }
 
-/* Euler, AB2, AB3 */
+/* Euler, AB2, AB3.  The reduced-precision builds need 196-256 registers: a
+ * few more would put one wave on a SIMD instead of two. */
+#define FVC_GEN_WAVES(MODE) ((MODE) == P_F64 ? 1 : 2)
 template <int MODE, int DIM, int UNS>
-__global__ __launch_bounds__(BLOCK) void k_advect_gen(DevMesh m, DevField f, PtrSet p, const int *__restrict__ index,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_GEN_WAVES(MODE)))) void k_advect_gen(DevMesh m, DevField f, PtrSet p, const int *__restrict__ index,
                                                      int64_t begin, int64_t count, double t1, double t2, int itype,
                                                      double dt, int extrap, ErrBuf eb, unsigned long long *steps) {
     advect_body<MODE, DIM, UNS, 1>(m, f, p, index, begin, count, t1, t2, itype, dt, extrap, eb, steps);
@@ -1315,7 +1315,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_RK4_W
 }
 
 template <int MODE, int DIM, int UNS>
-__global__ __launch_bounds__(BLOCK) void k_ftle_advect_gen(DevMesh m, DevField f, FtleDev d,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_GEN_WAVES(MODE)))) void k_ftle_advect_gen(DevMesh m, DevField f, FtleDev d,
                                                           const int *__restrict__ active, int64_t nactive, double t1,
                                                           double t2, int itype, double dt, int extrap, ErrBuf eb,
                                                           unsigned long long *steps) {
