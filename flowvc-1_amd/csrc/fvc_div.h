@@ -7,7 +7,7 @@
  * rounded to nearest (P. Markstein, Computation of elementary functions on
  * the IBM RISC System/6000 processor, 1990).  Five instructions where a
  * division takes twelve and more.  It holds for finite quotients and
- * residuals clear of the ends of the range: b in [1e-100, 1e100] (callers
+ * residuals clear of the ends of the range: |b| in [1e-100, 1e100] (callers
  * keep y = 0 for others and divide); |a| under about 2^-900 may miss the last
  * bit, an infinite a gives NaN (callers test for it).  Compiled for the
  * device and, by the tests, for the host. */
@@ -22,7 +22,9 @@
 #define FVC_DIV_HD
 #endif
 
-static inline FVC_DIV_HD double fvc_near_inverse(double b) { return b > 1e-100 && b < 1e100 ? 1.0 / b : 0.0; }
+static inline FVC_DIV_HD double fvc_near_inverse(double b) {
+    return fabs(b) > 1e-100 && fabs(b) < 1e100 ? 1.0 / b : 0.0;
+}
 
 static inline FVC_DIV_HD double fvc_div_near(double a, double b, double y) {
     double q = a * y;

@@ -25,7 +25,7 @@ int main(int argc, char **argv) {
     const double fixed[] = {6.0,  0.02, 0.5,    0.01,     0.1,           2.0 / 255, 1.0 / 127, 2.5 / 79, 1.0 / 3,
                             1e-3, 3.0,  1e-99, 9.9e99, 0x1.fffffffffffffp0, 0x1.0000000000001p0, 0x1.fffffffffffffp-7};
     for (unsigned i = 0; i < sizeof fixed / sizeof *fixed; i++) b[nb++] = fixed[i];
-    while (nb < 96) b[nb++] = ldexp(1.0 + unit(), (int)(rnd() % 60) - 40);
+    while (nb < 96) b[nb++] = ldexp(1.0 + unit(), (int)(rnd() % 60) - 40) * ((nb & 1) ? -1.0 : 1.0);
     long n = 0, bad = 0;
     for (int k = 0; k < nb; k++) {
         const double d = b[k], y = fvc_near_inverse(d);
@@ -50,7 +50,8 @@ int main(int argc, char **argv) {
         }
     }
     const int ranged = fvc_near_inverse(0.0) == 0.0 && fvc_near_inverse(1e-320) == 0.0 && fvc_near_inverse(1e200) == 0.0 &&
-                       fvc_near_inverse(-1.0) == 0.0 && fvc_near_inverse(NAN) == 0.0;
+                       fvc_near_inverse(-1e200) == 0.0 && fvc_near_inverse(INFINITY) == 0.0 &&
+                       fvc_near_inverse(NAN) == 0.0;
     printf("%ld %ld %d\n", n, bad, ranged);
     return 0;
 }
