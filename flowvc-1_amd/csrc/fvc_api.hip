@@ -67,6 +67,58 @@ int side_sync(fvc_ctx *c) {
     return hipStreamSynchronize(c->side) == hipSuccess ? FVC_OK : FVC_E_HIP;
 }
 
+/* pinned staging memory: copies from STAGE_MIN on go through it, in rounds of
+ * at most STAGE_MAX */
+constexpr size_t STAGE_MIN = (size_t)4 << 20, STAGE_MAX = (size_t)64 << 20, CHUNK = (size_t)8 << 20;
+
+/* the pinned staging buffer, at least `want` (<= STAGE_MAX) bytes; false when
+ * it cannot be had */
+static bool grow_stage(fvc_ctx *c, size_t want) {
+    if (c->stage && c->stage_bytes >= want) return true;
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
+    if (c->stage) hipHostFree(c->stage);
+    c->stage = nullptr;
+    c->stage_bytes = 0;
+    want = std::max(want, (size_t)1 << 20);
+    if (hipHostMalloc((void **)&c->stage, want, hipHostMallocDefault) != hipSuccess) {
+        c->stage = nullptr;
+        return false;
+    }
+    c->stage_bytes = want;
+    return true;
+}
+
+/* the device buffer that records are packed in, at least `want` bytes */
+static int grow_pack(fvc_ctx *c, size_t want) {
+    if (c->pack_bytes >= want) return FVC_OK;
+    FVC_HIP(hipStreamSynchronize(c->stream));
+    if (c->pack) hipFree(c->pack);
+    c->pack = nullptr;
+    c->pack_bytes = 0;
+    FVC_HIP(hipMalloc((void **)&c->pack, want));
+    c->pack_bytes = want;
+    return FVC_OK;
+}
+
+/* memcpy over up to 8 host threads, one for each 512 KB */
+static void host_copy(void *dst, const void *src, size_t bytes) {
+    const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
+    const int nthr = (int)std::min<size_t>({8, std::max(1u, hw / 2), std::max<size_t>(1, bytes >> 19)});
+    auto part = [&](int t) {
+        const size_t lo = (bytes * t / nthr) & ~(size_t)63, hi = t + 1 == nthr ? bytes : (bytes * (t + 1) / nthr) & ~(size_t)63;
+        memcpy((char *)dst + lo, (const char *)src + lo, hi - lo);
+    };
+    std::vector<std::thread> pool;
+    try {
+        for (int t = 1; t < nthr; t++) pool.emplace_back(part, t);
+    } catch (...) { /* fewer threads: the calling thread copies the rest */
+    }
+    const int started = (int)pool.size() + 1;
+    part(0);
+    for (int t = started; t < nthr; t++) part(t);
+    for (auto &th : pool) th.join();
+}
+
 /* Device -> host copy of a large block into caller (pageable) memory.  The
  * runtime moves pageable destinations through its own small staging buffer,
  * about 12 GB/s on a 168 MB copy; DMA into pinned memory runs at the link's
@@ -79,19 +131,8 @@ int side_sync(fvc_ctx *c) {
  * had, are only enqueued on the stream as a direct copy: the caller
  * synchronises the stream before reading them. */
 int copy_to_host(fvc_ctx *c, void *dst, const void *src, size_t bytes) {
-    constexpr size_t STAGE_MIN = (size_t)4 << 20, STAGE_MAX = (size_t)64 << 20, CHUNK = (size_t)8 << 20;
     if (bytes == 0) return FVC_OK;
-    if (bytes >= STAGE_MIN && c->stage_bytes < std::min(bytes, STAGE_MAX)) {
-        if (hipStreamSynchronize(c->stream) != hipSuccess) return FVC_E_HIP;
-        if (c->stage) hipHostFree(c->stage);
-        c->stage = nullptr;
-        c->stage_bytes = 0;
-        const size_t want = std::min(bytes, STAGE_MAX);
-        if (hipHostMalloc((void **)&c->stage, want, hipHostMallocDefault) == hipSuccess)
-            c->stage_bytes = want;
-        else
-            c->stage = nullptr;
-    }
+    if (bytes >= STAGE_MIN && !grow_stage(c, std::min(bytes, STAGE_MAX))) (void)hipGetLastError();
     if (bytes < STAGE_MIN || !c->stage) {
         FVC_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
         return FVC_OK;
@@ -459,6 +500,9 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
             return FVC_E_HIP;
         }
     }
+    /* the staging that every output of up to STAGE_MIN bytes goes through, here
+     * and not in the first pass (pinning takes about 0.2 ms) */
+    if (!grow_stage(c, STAGE_MIN)) (void)hipGetLastError();
     if (hipMemset(c->d_status, 0, sizeof(fvc_status)) != hipSuccess) {
         fvc_destroy(c);
         return FVC_E_HIP;
@@ -578,6 +622,7 @@ extern "C" void fvc_destroy(fvc_ctx *c) {
         if (s) hipFree(s);
     if (c->cet_lo) hipFree(c->cet_lo);
     if (c->cet_enc) hipFree(c->cet_enc);
+    if (c->pack) hipFree(c->pack);
     hipFree(c->X64);
     hipFree(c->ER);
     hipFree(c->conn);
@@ -906,46 +951,157 @@ extern "C" int fvc_particles_set(fvc_particles *p, int64_t begin, const fvc_poin
     return FVC_OK;
 }
 
-extern "C" int fvc_particles_get(fvc_particles *p, int64_t begin, fvc_point *recs, int64_t n) {
-    if (!p || !p->ctx || !recs || begin < 0 || n < 0 || begin + n > p->cap) return FVC_E_INVALID;
-    fvc_ctx *c = p->ctx;
-    std::vector<double> d(8 * (size_t)n);
-    std::vector<int> iv(3 * (size_t)n);
-    double *src[8] = {p->X[0], p->X[1], p->X[2], p->V[0], p->V[1], p->V[2], p->left_time, p->scalar};
-    int rc = FVC_OK;
-    for (int a = 0; a < 8 && !rc; a++) rc = copy_to_host(c, d.data() + a * n, src[a] + begin, 8 * (size_t)n);
-    int *isrc[3] = {p->elem, p->aux, p->left};
-    for (int a = 0; a < 3 && !rc; a++) rc = copy_to_host(c, iv.data() + a * n, isrc[a] + begin, 4 * (size_t)n);
-    if (rc) return rc;
-    FVC_HIP(hipStreamSynchronize(c->stream));
-    for (int64_t i = 0; i < n; i++) {
-        for (int a = 0; a < 3; a++) {
-            recs[i].X[a] = d[a * n + i];
-            recs[i].V[a] = d[(3 + a) * n + i];
-        }
-        recs[i].LeftDomainTime = d[6 * n + i];
-        recs[i].Scalar = d[7 * n + i];
-        recs[i].ElementIndex = iv[i];
-        recs[i].AuxElementIndex = iv[n + i];
-        recs[i].LeftDomain = iv[2 * n + i];
-        recs[i].pad_ = 0;
+/* ------------------------------------------------------------------------ */
+/* records on their way out                                                  */
+/* ------------------------------------------------------------------------ */
+/* The device keeps particle state by component; callers get it by record.
+ * A kernel packs the records, and the host only copies: interleaving on the
+ * host took one thread 25 ns a record, after a copy of every component into
+ * fresh pageable memory (4M positions: 28 ms of a 60 ms pass).  A record is
+ * written as 16-byte parts, one a lane, so that a wave's stores are
+ * contiguous; the scattered component reads stay in the L2. */
+struct PackPoints {
+    const double *X[3], *V[3], *lt, *scalar; /* null: zero */
+    const int *elem, *aux, *left;            /* null elem / aux: zero */
+};
+
+__global__ __launch_bounds__(256) void k_pack_points(PackPoints s, int64_t n, double2 *__restrict__ out) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 5 * n) return;
+    const int64_t i = t / 5;
+    const int part = (int)(t - 5 * i);
+    double2 v = make_double2(0.0, 0.0);
+    if (part == 0) v = make_double2(s.X[0][i], s.X[1][i]);
+    else if (part == 1) v = make_double2(s.X[2] ? s.X[2][i] : 0.0, s.V[0] ? s.V[0][i] : 0.0);
+    else if (part == 2) v = s.V[0] ? make_double2(s.V[1][i], s.V[2][i]) : v;
+    else if (part == 3) v = make_double2(__hiloint2double(s.aux ? s.aux[i] : 0, s.elem ? s.elem[i] : 0),
+                                         __hiloint2double(0, s.left[i]));
+    else v = make_double2(s.lt[i], s.scalar ? s.scalar[i] : 0.0);
+    out[t] = v;
+}
+
+__global__ __launch_bounds__(256) void k_pack_xyz(const double *__restrict__ x, const double *__restrict__ y,
+                                                  const double *__restrict__ z, int64_t n, double *__restrict__ out) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 3 * n) return;
+    const int64_t i = t / 3;
+    const int a = (int)(t - 3 * i);
+    out[t] = a == 0 ? x[i] : a == 1 ? y[i] : z[i];
+}
+
+/* n records of rec bytes to dst: pack(begin, count, device pointer) enqueues
+ * the kernel that writes `count` of them from `begin` on.  Up to STAGE_MIN
+ * bytes (latency counts) straight into the pinned buffer, one launch and one
+ * wait; more in rounds through a device buffer and copy_to_host.  `more`
+ * further bytes follow in the same wait, from `src2` on the device. */
+template <class F>
+static int out_records(fvc_ctx *c, void *dst, int64_t n, size_t rec, F pack, void *dst2 = nullptr,
+                       const void *src2 = nullptr, size_t more = 0) {
+    const size_t total = rec * (size_t)n, at2 = (total + 255) & ~(size_t)255;
+    if (at2 + more <= STAGE_MIN && grow_stage(c, at2 + more)) {
+        pack((int64_t)0, n, c->stage);
+        FVC_HIP(hipGetLastError());
+        if (more) FVC_HIP(hipMemcpyAsync(c->stage + at2, src2, more, hipMemcpyDeviceToHost, c->stream));
+        FVC_HIP(hipStreamSynchronize(c->stream));
+        host_copy(dst, c->stage, total);
+        if (more) memcpy(dst2, c->stage + at2, more);
+        return FVC_OK;
+    }
+    const int64_t round = std::min<int64_t>(n, (int64_t)(STAGE_MAX / rec));
+    int rc0 = grow_pack(c, rec * (size_t)round);
+    if (rc0) return rc0;
+    for (int64_t b = 0; b < n; b += round) {
+        const int64_t k = std::min(round, n - b);
+        pack(b, k, c->pack);
+        FVC_HIP(hipGetLastError());
+        int rc = copy_to_host(c, (char *)dst + rec * (size_t)b, c->pack, rec * (size_t)k);
+        if (rc) return rc;
+        FVC_HIP(hipStreamSynchronize(c->stream));
+    }
+    if (more) {
+        int rc = copy_to_host(c, dst2, src2, more);
+        if (rc) return rc;
+        FVC_HIP(hipStreamSynchronize(c->stream));
     }
     return FVC_OK;
+}
+
+static int out_points(fvc_ctx *c, fvc_point *recs, int64_t n, const PackPoints &src) {
+    return out_records(c, recs, n, sizeof(fvc_point), [&](int64_t b, int64_t k, char *to) {
+        PackPoints s = src;
+        for (int a = 0; a < 3; a++) {
+            if (s.X[a]) s.X[a] += b;
+            if (s.V[a]) s.V[a] += b;
+        }
+        s.lt += b;
+        if (s.scalar) s.scalar += b;
+        if (s.elem) s.elem += b;
+        if (s.aux) s.aux += b;
+        s.left += b;
+        k_pack_points<<<(unsigned)((5 * k + 255) / 256), 256, 0, c->stream>>>(s, k, (double2 *)to);
+    });
+}
+
+extern "C" int fvc_particles_get(fvc_particles *p, int64_t begin, fvc_point *recs, int64_t n) {
+    if (!p || !p->ctx || !recs || begin < 0 || n < 0 || begin + n > p->cap) return FVC_E_INVALID;
+    if (n == 0) return FVC_OK;
+    const PackPoints s{{p->X[0] + begin, p->X[1] + begin, p->X[2] + begin},
+                       {p->V[0] + begin, p->V[1] + begin, p->V[2] + begin},
+                       p->left_time + begin,
+                       p->scalar + begin,
+                       p->elem + begin,
+                       p->aux + begin,
+                       p->left + begin};
+    return out_points(p->ctx, recs, n, s);
+}
+
+/* n particles from src to dst, all components in one launch (18 copies, one
+ * a component, cost 4-6 us each before their bytes counted) */
+struct CopyArrays {
+    double *dd[14];
+    const double *ds[14];
+    int *id[4];
+    const int *is[4];
+};
+
+__global__ __launch_bounds__(256) void k_copy_particles(CopyArrays a, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double d[14];
+    int v[4];
+    for (int k = 0; k < 14; k++) d[k] = a.ds[k][i];
+    for (int k = 0; k < 4; k++) v[k] = a.is[k][i];
+    for (int k = 0; k < 14; k++) a.dd[k][i] = d[k];
+    for (int k = 0; k < 4; k++) a.id[k][i] = v[k];
 }
 
 static int particles_d2d(fvc_particles *dst, int64_t db, const fvc_particles *src, int64_t sb, int64_t n) {
     fvc_ctx *c = dst->ctx;
     dst->act_begin = -1; /* copied-in state may bring particles back */
-    double *ds[8] = {dst->X[0], dst->X[1], dst->X[2], dst->V[0], dst->V[1], dst->V[2], dst->left_time, dst->scalar};
-    double *ss[8] = {src->X[0], src->X[1], src->X[2], src->V[0], src->V[1], src->V[2], src->left_time, src->scalar};
-    for (int a = 0; a < 8; a++)
-        FVC_HIP(hipMemcpyAsync(ds[a] + db, ss[a] + sb, 8 * n, hipMemcpyDeviceToDevice, c->stream));
-    int *di[4] = {dst->elem, dst->aux, dst->left, dst->nhist};
-    int *si[4] = {src->elem, src->aux, src->left, src->nhist};
-    for (int a = 0; a < 4; a++)
-        FVC_HIP(hipMemcpyAsync(di[a] + db, si[a] + sb, 4 * n, hipMemcpyDeviceToDevice, c->stream));
-    for (int a = 0; a < 6; a++)
-        FVC_HIP(hipMemcpyAsync(dst->H[a] + db, src->H[a] + sb, 8 * n, hipMemcpyDeviceToDevice, c->stream));
+    double *dd[14] = {dst->X[0], dst->X[1], dst->X[2], dst->V[0], dst->V[1], dst->V[2], dst->left_time, dst->scalar,
+                      dst->H[0], dst->H[1], dst->H[2], dst->H[3], dst->H[4], dst->H[5]};
+    double *ds[14] = {src->X[0], src->X[1], src->X[2], src->V[0], src->V[1], src->V[2], src->left_time, src->scalar,
+                      src->H[0], src->H[1], src->H[2], src->H[3], src->H[4], src->H[5]};
+    int *id[4] = {dst->elem, dst->aux, dst->left, dst->nhist};
+    int *is[4] = {src->elem, src->aux, src->left, src->nhist};
+    if (dst == src && db < sb + n && sb < db + n) { /* overlapping ranges of one set: component by component */
+        for (int a = 0; a < 14; a++)
+            FVC_HIP(hipMemcpyAsync(dd[a] + db, ds[a] + sb, 8 * n, hipMemcpyDeviceToDevice, c->stream));
+        for (int a = 0; a < 4; a++)
+            FVC_HIP(hipMemcpyAsync(id[a] + db, is[a] + sb, 4 * n, hipMemcpyDeviceToDevice, c->stream));
+    } else {
+        CopyArrays a;
+        for (int k = 0; k < 14; k++) {
+            a.dd[k] = dd[k] + db;
+            a.ds[k] = ds[k] + sb;
+        }
+        for (int k = 0; k < 4; k++) {
+            a.id[k] = id[k] + db;
+            a.is[k] = is[k] + sb;
+        }
+        k_copy_particles<<<(unsigned)((n + 255) / 256), 256, 0, c->stream>>>(a, n);
+        FVC_HIP(hipGetLastError());
+    }
     FVC_HIP(hipStreamSynchronize(c->stream));
     return FVC_OK;
 }
@@ -959,15 +1115,15 @@ extern "C" int fvc_particles_copy(fvc_particles *dst, int64_t db, const fvc_part
 
 extern "C" int fvc_particles_get_xyz(fvc_particles *p, int64_t begin, double *xyz, int32_t *left, int64_t n) {
     if (!p || !p->ctx || !xyz || begin < 0 || n < 0 || begin + n > p->cap) return FVC_E_INVALID;
+    if (n == 0) return FVC_OK;
     fvc_ctx *c = p->ctx;
-    std::vector<double> d(3 * (size_t)n);
-    for (int a = 0; a < 3; a++)
-        FVC_HIP(hipMemcpyAsync(d.data() + a * n, p->X[a] + begin, 8 * n, hipMemcpyDeviceToHost, c->stream));
-    if (left) FVC_HIP(hipMemcpyAsync(left, p->left + begin, 4 * n, hipMemcpyDeviceToHost, c->stream));
-    FVC_HIP(hipStreamSynchronize(c->stream));
-    for (int64_t i = 0; i < n; i++)
-        for (int a = 0; a < 3; a++) xyz[3 * i + a] = d[a * n + i];
-    return FVC_OK;
+    return out_records(
+        c, xyz, n, 3 * sizeof(double),
+        [&](int64_t b, int64_t k, char *to) {
+            k_pack_xyz<<<(unsigned)((3 * k + 255) / 256), 256, 0, c->stream>>>(
+                p->X[0] + begin + b, p->X[1] + begin + b, p->X[2] + begin + b, k, (double *)to);
+        },
+        left, p->left + begin, left ? sizeof(int) * (size_t)n : 0);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -1154,6 +1310,46 @@ extern "C" int fvc_locate_noalloc(fvc_ctx *c, const double *xyz, const int32_t *
     return FVC_OK;
 }
 
+/* records of located seeds (k_pack_points' layout): positions from the list
+ * (z = 0 in 2-D, tracers.c:1033) or the grid */
+struct SeedPack {
+    int chain, dims, mesh_type;
+    const double *xyz;
+    double mn[3], del[3];
+    int res[3];
+    const int *elem, *left;
+    const double *lt;
+};
+
+__global__ __launch_bounds__(256) void k_pack_seeds(SeedPack s, int64_t begin, int64_t n, double2 *__restrict__ out) {
+#pragma clang fp contract(off)
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 5 * n) return;
+    const int64_t i = begin + t / 5;
+    const int part = (int)(t % 5);
+    double2 v = make_double2(0.0, 0.0);
+    if (part < 2) {
+        double X[3];
+        if (s.chain == 0) {
+            for (int a = 0; a < 3; a++) X[a] = s.xyz[3 * i + a];
+            if (s.dims == 2) X[2] = 0.0;
+        } else {
+            const int64_t plane = (int64_t)s.res[0] * s.res[1];
+            const int ii = (int)(i % s.res[0]), jj = (int)((i / s.res[0]) % s.res[1]), kk = (int)(i / plane);
+            X[0] = s.mn[0] + ii * s.del[0];
+            X[1] = s.mn[1] + jj * s.del[1];
+            X[2] = s.mn[2] + kk * s.del[2];
+        }
+        v = part == 0 ? make_double2(X[0], X[1]) : make_double2(X[2], 0.0);
+    } else if (part == 3) {
+        const int e = s.elem[i], l = s.left[i];
+        v = make_double2(__hiloint2double(s.chain == 0 && !l ? e : 0, s.mesh_type == 1 ? e : 0), __hiloint2double(0, l));
+    } else if (part == 4) {
+        v.x = s.lt[i];
+    }
+    out[t] = v;
+}
+
 static int seed_common(fvc_ctx *c, int chain, const double *xyz, int64_t n, const double mn[3], const double del[3],
                        const int32_t res[3], int lsc, fvc_point *out) {
 #pragma clang fp contract(off)
@@ -1168,30 +1364,15 @@ static int seed_common(fvc_ctx *c, int chain, const double *xyz, int64_t n, cons
     FVC_HIP(hipMallocAsync((void **)&dl, sizeof(int) * n, c->stream));
     int rc = launch_seed_chain(c, chain, n, dx, mn, del, res, lsc, de, dl, dlt);
     if (!rc) {
-        std::vector<int> e(n), l(n);
-        std::vector<double> lt(n);
-        FVC_HIP(hipMemcpyAsync(e.data(), de, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
-        FVC_HIP(hipMemcpyAsync(l.data(), dl, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
-        FVC_HIP(hipMemcpyAsync(lt.data(), dlt, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-        FVC_HIP(hipStreamSynchronize(c->stream));
-        for (int64_t i = 0; i < n; i++) {
-            fvc_point &p = out[i];
-            memset(&p, 0, sizeof p);
-            if (chain == 0) {
-                p.X[0] = xyz[3 * i];
-                p.X[1] = xyz[3 * i + 1];
-                p.X[2] = c->mesh.dims == 2 ? 0.0 : xyz[3 * i + 2];
-            } else {
-                int ii = (int)(i % res[0]), jj = (int)((i / res[0]) % res[1]), kk = (int)(i / ((int64_t)res[0] * res[1]));
-                p.X[0] = mn[0] + ii * del[0];
-                p.X[1] = mn[1] + jj * del[1];
-                p.X[2] = mn[2] + kk * del[2];
-            }
-            p.ElementIndex = c->mesh.mesh_type == 1 ? e[i] : 0;
-            p.AuxElementIndex = chain == 0 && !l[i] ? e[i] : 0;
-            p.LeftDomain = l[i];
-            p.LeftDomainTime = lt[i];
+        SeedPack s{chain, c->mesh.dims, c->mesh.mesh_type, dx, {0, 0, 0}, {0, 0, 0}, {1, 1, 1}, de, dl, dlt};
+        for (int a = 0; a < 3 && chain != 0; a++) {
+            s.mn[a] = mn[a];
+            s.del[a] = del[a];
+            s.res[a] = res[a];
         }
+        rc = out_records(c, out, n, sizeof(fvc_point), [&](int64_t b, int64_t k, char *to) {
+            k_pack_seeds<<<(unsigned)((5 * k + 255) / 256), 256, 0, c->stream>>>(s, b, k, (double2 *)to);
+        });
     }
     if (dx) hipFreeAsync(dx, c->stream);
     hipFreeAsync(dlt, c->stream);
@@ -1204,11 +1385,12 @@ static int seed_common(fvc_ctx *c, int chain, const double *xyz, int64_t n, cons
 extern "C" int fvc_seed_list(fvc_ctx *c, const double *xyz, int64_t n, int32_t lsc, fvc_point *out) {
     if (!c || !xyz || !out || n < 0) return FVC_E_INVALID;
     if (n == 0) return FVC_OK;
+    if (c->mesh.dims == 3) return seed_common(c, 0, xyz, n, nullptr, nullptr, nullptr, lsc, out);
     std::vector<double> x(3 * (size_t)n);
     for (int64_t i = 0; i < n; i++) {
         x[3 * i] = xyz[3 * i];
         x[3 * i + 1] = xyz[3 * i + 1];
-        x[3 * i + 2] = c->mesh.dims == 2 ? 0.0 : xyz[3 * i + 2]; /* tracers.c:1033 */
+        x[3 * i + 2] = 0.0; /* tracers.c:1033 */
     }
     return seed_common(c, 0, x.data(), n, nullptr, nullptr, nullptr, lsc, out);
 }
@@ -1424,6 +1606,19 @@ extern "C" void fvc_ftle_destroy(fvc_ftle *f) {
     delete f;
 }
 
+/* w: FTLEwT then FTLEwoT, n values each */
+__global__ __launch_bounds__(256) void k_ftle_restore(const int *__restrict__ have0, const double *__restrict__ w0,
+                                                      int64_t n, int *__restrict__ have, double *__restrict__ w,
+                                                      int *__restrict__ exited, int *__restrict__ advected) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    have[i] = have0[i];
+    w[i] = w0[i];
+    w[n + i] = w0[n + i];
+    exited[i] = 0;
+    advected[i] = 0;
+}
+
 extern "C" int fvc_ftle_reset(fvc_ftle *f) {
     if (!f || !f->ctx || !f->init_pts) return FVC_E_INVALID;
     fvc_ctx *c = f->ctx;
@@ -1432,10 +1627,9 @@ extern "C" int fvc_ftle_reset(fvc_ftle *f) {
     if (rc) return rc;
     rc = particles_d2d(f->pts, 0, f->init_pts, 0, f->n);
     if (rc) return rc;
-    FVC_HIP(hipMemcpyAsync(f->have, f->init_have, sizeof(int) * n, hipMemcpyDeviceToDevice, c->stream));
-    FVC_HIP(hipMemcpyAsync(f->wt, f->init_w, sizeof(double) * 2 * n, hipMemcpyDeviceToDevice, c->stream));
-    FVC_HIP(hipMemsetAsync(f->exited, 0, sizeof(int) * n, c->stream));
-    FVC_HIP(hipMemsetAsync(f->advected, 0, sizeof(int) * n, c->stream));
+    k_ftle_restore<<<(unsigned)((n + 255) / 256), 256, 0, c->stream>>>(f->init_have, f->init_w, (int64_t)n, f->have,
+                                                                       f->wt, f->exited, f->advected);
+    FVC_HIP(hipGetLastError());
     FVC_HIP(hipStreamSynchronize(c->stream));
     f->status = 0;
     return FVC_OK;
@@ -1471,32 +1665,47 @@ extern "C" int fvc_ftle_frame(fvc_ftle *f, int32_t dir, int32_t lo, int32_t hi, 
     return FVC_OK;
 }
 
-/* i-major storage (P = (i*r1 + j)*r2 + k) -> k, j, i file order (q = (k*r1 + j)*r0 + i) */
+/* i-major storage (P = (i*r1 + j)*r2 + k) -> values [begin, begin + n) of the
+ * k, j, i file order (q = (k*r1 + j)*r0 + i), wt then wot */
 __global__ void k_ftle_kji(const double *__restrict__ wt, const double *__restrict__ wot, int r0, int r1, int r2,
-                           double *__restrict__ out) {
-    const int64_t n = (int64_t)r0 * r1 * r2;
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
+                           int64_t begin, int64_t n, double *__restrict__ out) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const int64_t q = begin + t;
     const int i = (int)(q % r0), j = (int)((q / r0) % r1), k = (int)(q / ((int64_t)r0 * r1));
     const int64_t P = ((int64_t)i * r1 + j) * r2 + k;
-    out[q] = wt[P];
-    out[n + q] = wot[P];
+    out[t] = wt[P];
+    out[n + t] = wot[P];
 }
 
-/* FTLE values of a grid to host memory in the file order of ftle.c:1302-1315 */
+/* FTLE values of a grid to host memory in the file order of ftle.c:1302-1315:
+ * as out_records, but in two blocks */
 int fvc::copy_ftle_kji(fvc_ctx *c, const double *d_wt, const double *d_wot, const int32_t res[3], double *wt,
                        double *wot) {
-    const size_t n = (size_t)res[0] * res[1] * res[2];
-    double *tmp = nullptr;
-    FVC_HIP(hipMallocAsync((void **)&tmp, sizeof(double) * 2 * n, c->stream));
-    k_ftle_kji<<<(unsigned)((n + 255) / 256), 256, 0, c->stream>>>(d_wt, d_wot, res[0], res[1], res[2], tmp);
-    hipError_t e = hipGetLastError();
-    int rc = e == hipSuccess ? FVC_OK : FVC_E_HIP;
-    if (!rc && wt) rc = copy_to_host(c, wt, tmp, sizeof(double) * n);
-    if (!rc && wot) rc = copy_to_host(c, wot, tmp + n, sizeof(double) * n);
-    (void)hipFreeAsync(tmp, c->stream);
-    if (!rc) rc = hipStreamSynchronize(c->stream) == hipSuccess ? FVC_OK : FVC_E_HIP;
-    if (rc) c->last_error = std::string("FTLE output copy: ") + hipGetErrorString(hipGetLastError());
+    const int64_t n = (int64_t)res[0] * res[1] * res[2];
+    const size_t rec = 2 * sizeof(double);
+    auto pack = [&](int64_t b, int64_t k, void *to) {
+        k_ftle_kji<<<(unsigned)((k + 255) / 256), 256, 0, c->stream>>>(d_wt, d_wot, res[0], res[1], res[2], b, k,
+                                                                       (double *)to);
+    };
+    if (rec * (size_t)n <= STAGE_MIN && grow_stage(c, rec * (size_t)n)) {
+        pack(0, n, c->stage);
+        FVC_HIP(hipGetLastError());
+        FVC_HIP(hipStreamSynchronize(c->stream));
+        if (wt) host_copy(wt, c->stage, sizeof(double) * (size_t)n);
+        if (wot) host_copy(wot, (double *)c->stage + n, sizeof(double) * (size_t)n);
+        return FVC_OK;
+    }
+    const int64_t round = std::min<int64_t>(n, (int64_t)(STAGE_MAX / rec));
+    int rc = grow_pack(c, rec * (size_t)round);
+    for (int64_t b = 0; b < n && !rc; b += round) {
+        const int64_t k = std::min(round, n - b);
+        pack(b, k, c->pack);
+        FVC_HIP(hipGetLastError());
+        if (wt) rc = copy_to_host(c, wt + b, c->pack, sizeof(double) * (size_t)k);
+        if (!rc && wot) rc = copy_to_host(c, wot + b, (double *)c->pack + k, sizeof(double) * (size_t)k);
+        FVC_HIP(hipStreamSynchronize(c->stream));
+    }
     return rc;
 }
 

@@ -64,6 +64,10 @@ struct fvc_ctx {
      * demand, with one event per chunk */
     char *stage;
     size_t stage_bytes;
+    /* device buffer in which kernels pack records on their way out, grown on
+     * demand to at most OUT_ROUND bytes */
+    char *pack;
+    size_t pack_bytes;
     std::vector<hipEvent_t> stage_ev;
     /* side stream: an FTLE slide frame's early FTLE (from a snapshot of its
      * stencils) runs there beside the next frame's advection; side_done

@@ -77,3 +77,22 @@ def test_large_ftle_output_equals_a_narrow_grid_of_the_same_spacing():
     assert live.sum() > 500_000
     np.testing.assert_array_equal(Lt[live] * 2.0 == Lo[live], np.ones(live.sum(), bool))
     ctx.close()
+
+
+# 80-byte records: 52,428 fill the 4 MB that go out in one wait, 838,860 one
+# round of the packing buffer; 24-byte positions: 174,762 and 2,796,202
+@pytest.mark.parametrize("n", [5, 63, 52428, 52429, 174763, 838860, 838861, 1700001])
+def test_packed_records_and_positions_at_round_edges(n):
+    ctx = fvc.Context(2, [0.0, 1.0, 0.0, 1.0, 0.0, 0.0], "f64", 2, cart_min=[0.0] * 3, cart_max=[1.0, 1.0, 0.0],
+                      cart_res=[4, 4, 1])
+    recs = _records(n, 9)
+    p, q = fvc.Particles(ctx, n + 3), fvc.Particles(ctx, n + 3)
+    p.set(recs, begin=2)
+    print("packed records n %d" % n, flush=True)
+    assert _same_bytes(p.get(n, begin=2), recs)
+    xyz, left = p.get_xyz(n, begin=2)
+    np.testing.assert_array_equal(xyz, recs["X"])
+    np.testing.assert_array_equal(left, recs["LeftDomain"])
+    q.copy_from(p, n, begin=1, src_begin=2)
+    assert _same_bytes(q.get(n, begin=1), recs)
+    ctx.close()
