@@ -1444,6 +1444,7 @@ static int ftle_alloc(fvc_ctx *c, const double mn[3], const double del[3], const
     f->n = (int64_t)f->res[0] * f->res[1] * f->res[2];
     f->start_time = start_time;
     f->stop_time = stop_time;
+    f->nactive = -1;
     int rc = fvc_particles_create(c, f->n, &f->pts);
     if (rc) {
         fvc_ftle_destroy(f);
@@ -1632,6 +1633,7 @@ extern "C" int fvc_ftle_reset(fvc_ftle *f) {
     FVC_HIP(hipGetLastError());
     FVC_HIP(hipStreamSynchronize(c->stream));
     f->status = 0;
+    f->nactive = -1;
     return FVC_OK;
 }
 

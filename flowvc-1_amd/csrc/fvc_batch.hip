@@ -396,7 +396,7 @@ static BatchDev batch_dev(fvc_batch *b, int k, int parity) {
     d.n_in = b->counts + 2 * k + parity;
     d.n_out = b->counts + 2 * k + (parity ^ 1);
     d.queue = b->queue + NQ * k;
-    d.steps = b->ctx->d_steps;
+    d.steps = b->ctx->d_steps + 2;
     d.err = b->ctx->d_err;
     d.where = b->ctx->d_where;
     return d;
@@ -687,7 +687,7 @@ extern "C" int fvc_batch_run(fvc_batch *b, const fvc_batch_params *bp, int64_t *
     const int grid[2] = {grid_for_batch(b, 0, bs, bp->waves_per_cu), grid_for_batch(b, 1, bs, bp->waves_per_cu)};
     /* every launch takes at least one budget unit from each active particle */
     const int64_t max_rounds = b->max_budget / std::min<int64_t>(budget, b->max_budget) + 2;
-    FVC_HIP(hipMemsetAsync(c->d_steps, 0, sizeof(unsigned long long), c->stream));
+    FVC_HIP(hipMemsetAsync(c->d_steps + 2, 0, sizeof(unsigned long long), c->stream));
     timing_begin(c); /* with timing on: device time of the whole run */
     int rc0 = launch_releases(b);
     if (rc0) return rc0;
@@ -734,8 +734,7 @@ extern "C" int fvc_batch_run(fvc_batch *b, const fvc_batch_params *bp, int64_t *
     }
     timing_end(c);
     int rc = check_err(c, "fvc_batch_run");
-    unsigned long long st = 0;
-    if (hipMemcpy(&st, c->d_steps, sizeof st, hipMemcpyDeviceToHost) != hipSuccess && !rc) rc = FVC_E_HIP;
+    const unsigned long long st = c->h_status->steps[2];
     c->last_steps = (int64_t)st;
     timing_collect(c, (int64_t)st);
     if (particle_steps) *particle_steps = (int64_t)st;

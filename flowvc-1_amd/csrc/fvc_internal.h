@@ -15,7 +15,9 @@
 
 /* what the kernels report to the host after a launch */
 struct fvc_status {
-    unsigned long long steps[2]; /* particle-steps; idle lanes (fvc_advect) */
+    /* particle-steps and idle lanes of the advection launches, never cleared
+     * (take_steps takes the differences); particle-steps of batches and servers */
+    unsigned long long steps[3];
     int64_t where;               /* point of the first error */
     int err;                     /* first error code, 0 if none */
     int count;                   /* length of the last compacted list */
@@ -53,6 +55,7 @@ struct fvc_ctx {
     int *d_err;
     int64_t *d_where;
     unsigned long long *d_steps;
+    unsigned long long steps_seen[2]; /* steps[0], steps[1] when last taken */
     int64_t last_steps;
     int64_t last_idle; /* lanes of the last fvc_advect launch whose particle was not integrated */
     std::string last_error;
@@ -128,7 +131,9 @@ struct fvc_ftle {
     double *Vn[3];
     int *active;    /* compacted indices of points to integrate (Z-ordered) */
     int *zperm;     /* grid points in Z-order */
-    int64_t nactive;
+    int64_t nactive;     /* length of `active`, -1: to be built */
+    int active_extrap;   /* the extrapolation flag it was built for */
+    int64_t active_gone; /* points on it that had left when the last frame began */
     /* stencil snapshots of the early FTLE, used by alternate frames */
     void *snap[2];
     int64_t snap_cap;
@@ -179,6 +184,7 @@ struct FtleDev {
     double *Xn[3], *Vn[3];
     int *elem_new, *exited, *advected;
     double *exit_time;
+    int *early_nt = nullptr; /* counter of triggered points that the frame's advection clears */
 };
 FtleDev ftle_dev(fvc_ftle *f);
 
@@ -218,6 +224,12 @@ int launch_copy_probe(fvc_ctx *c, void *dst, const void *src, int64_t bytes);
 int copy_ftle_kji(fvc_ctx *c, const double *d_wt, const double *d_wot, const int32_t res[3], double *wt, double *wot);
 
 int check_err(fvc_ctx *c, const char *what);
+/* after check_err: last_steps and last_idle of the launches since the last call */
+inline void take_steps(fvc_ctx *c) {
+    c->last_steps = (int64_t)(c->h_status->steps[0] - c->steps_seen[0]);
+    c->last_idle = (int64_t)(c->h_status->steps[1] - c->steps_seen[1]);
+    for (int k = 0; k < 2; k++) c->steps_seen[k] = c->h_status->steps[k];
+}
 /* order the main stream after the side stream's last launch / wait for it on the host */
 int side_join(fvc_ctx *c);
 int side_sync(fvc_ctx *c);

@@ -297,7 +297,6 @@ __global__ __launch_bounds__(BLOCK) void k_advect_times_gen(DevMesh m, DevField 
 
 int launch_advect_times(fvc_ctx *c, PtrSet p, int64_t begin, int64_t count, const double *dtt, const DevField &f,
                         const fvc_int_params &ip) {
-    FVC_HIP(hipMemsetAsync(c->d_steps, 0, sizeof(unsigned long long), c->stream));
     if (count > 0) {
         if (ip.int_type == FVC_INT_RK4 && !f.sr_lo && !f.cet_lo)
             FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_advect_times_rk4,
@@ -312,7 +311,7 @@ int launch_advect_times(fvc_ctx *c, PtrSet p, int64_t begin, int64_t count, cons
         FVC_HIP(hipGetLastError());
     }
     int rc = check_err(c, "fvc_advect_times");
-    c->last_steps = (int64_t)c->h_status->steps[0];
+    take_steps(c);
     return rc;
 }
 
@@ -351,7 +350,6 @@ int launch_active_list(fvc_ctx *c, PtrSet p, int64_t begin, int64_t count, int e
  * indices relative to begin */
 int launch_advect(fvc_ctx *c, PtrSet p, const int *index, int64_t begin, int64_t count, double t1, double t2,
                   const DevField &f, const fvc_int_params &ip) {
-    FVC_HIP(hipMemsetAsync(c->d_steps, 0, 2 * sizeof(unsigned long long), c->stream));
     if (count > 0) {
         int block = ip.block > 0 ? ip.block : BLOCK;
         if (block != BLOCK) block = BLOCK; /* kernels are compiled for 256-lane blocks */
@@ -371,8 +369,7 @@ int launch_advect(fvc_ctx *c, PtrSet p, const int *index, int64_t begin, int64_t
         FVC_HIP(hipGetLastError());
     }
     int rc = check_err(c, "fvc_advect");
-    c->last_steps = (int64_t)c->h_status->steps[0];
-    c->last_idle = (int64_t)c->h_status->steps[1];
+    take_steps(c);
     if (count > 0) timing_collect(c, c->last_steps);
     return rc;
 }
@@ -1284,26 +1281,32 @@ __device__ __forceinline__ void ftle_advect_body(const DevMesh &m, const DevFiel
                                                  unsigned long long *steps) {
     int64_t q = xcd_block() * blockDim.x + threadIdx.x;
     uint32_t ns = 0;
+    bool idle = false;
+    if (q == 0 && d.early_nt) *d.early_nt = 0;
     if (q < nactive) {
         int64_t i = active[q];
-        PState s;
-        load_state(d.p, i, s, false, extrap);
-        int err = 0;
-        advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, extrap, err, ns,
-                                    sm_rows<MODE, DIM, UNS, GEN, BLOCK>());
-        if (err) raise_err(eb, err, i);
-        d.advected[i] = 1;
-        int ex = s.left && !extrap;
-        d.exited[i] = ex;
-        d.exit_time[i] = s.left_time;
-        for (int c = 0; c < 3; c++) {
-            d.Xn[c][i] = s.X[c];
-            if (extrap) d.Vn[c][i] = s.V[c];
+        if (!particle_live(d.p, i, extrap)) { /* left since the list was built */
+            idle = true;
+        } else {
+            PState s;
+            load_state(d.p, i, s, false, extrap);
+            int err = 0;
+            advect<MODE, DIM, UNS, GEN>(m, f, s, t1, t2, itype, dt, extrap, err, ns,
+                                        sm_rows<MODE, DIM, UNS, GEN, BLOCK>());
+            if (err) raise_err(eb, err, i);
+            d.advected[i] = 1;
+            int ex = s.left && !extrap;
+            d.exited[i] = ex;
+            d.exit_time[i] = s.left_time;
+            for (int c = 0; c < 3; c++) {
+                d.Xn[c][i] = s.X[c];
+                if (extrap) d.Vn[c][i] = s.V[c];
+            }
+            d.elem_new[i] = s.elem;
+            if (extrap) d.p.left[i] = s.left;
         }
-        d.elem_new[i] = s.elem;
-        if (extrap) d.p.left[i] = s.left;
     }
-    add_steps<MODE, DIM, UNS, GEN, false>(steps, ns);
+    add_steps<MODE, DIM, UNS, GEN, true>(steps, ns, idle);
 }
 
 template <int MODE, int DIM, int UNS>
@@ -1460,47 +1463,49 @@ __device__ inline int64_t early_trigger(const FtleDev &d, int64_t P, const int64
     return trig;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_early_flag(FtleDev d, int64_t n, int *__restrict__ flags) {
+/* The frame's triggered points, in any order (each one's early FTLE is its
+ * own), counted in *nt; with SNAP the stencil snapshot (EarlySnap) of the
+ * first cap of them.  One launch where flags, a stable compaction and a
+ * snapshot kernel took five (44 us a frame on 131,072 points, mostly
+ * launches); the waves that trigger nothing, nearly all, only read. */
+template <int SNAP>
+__global__ __launch_bounds__(BLOCK) void k_early_list(FtleDev d, int64_t n, int *__restrict__ list,
+                                                      int *__restrict__ nt, EarlySnap s) {
     const int64_t P = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (P >= n) return;
-    int fl = 0;
-    if (!d.have[P]) {
-        int cc[3];
-        int64_t nb[6];
-        bool has[6];
-        grid_nbrs(d, P, cc, nb, has);
-        fl = early_trigger(d, P, nb, has) != INT64_MAX;
-    }
-    flags[P] = fl;
-}
-
-/* the stencil snapshot of the first cap triggered points (EarlySnap) */
-__global__ __launch_bounds__(BLOCK) void k_early_snap(FtleDev d, const int *__restrict__ list,
-                                                     const int *__restrict__ d_nt, EarlySnap s) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int nt = *d_nt;
-    if (t == 0) *s.nt = nt;
-    if (t >= nt || t >= s.cap) return;
-    const int64_t P = list[t];
-    int cc[3];
-    int64_t nb[6];
+    int64_t nb[6], trig = INT64_MAX;
     bool has[6];
-    grid_nbrs(d, P, cc, nb, has);
-    const int64_t trig = early_trigger(d, P, nb, has);
-    s.P[t] = (int)P;
-    s.te[t] = d.exit_time[trig];
-    for (int q = 0; q < 7; q++) {
-        const int64_t idx = q < 6 ? nb[q] : P;
-        const bool ok = q == 6 || has[q];
-        for (int c = 0; c < 3; c++) s.X[(q * 3 + c) * s.cap + t] = ok ? d.p.X[c][idx] : 0.0;
-        int left = 0, elem = -1;
-        if (ok) {
-            left = d.p.left[idx];
-            const bool updated = idx < trig && d.advected[idx] && !d.exited[idx];
-            elem = updated ? d.elem_new[idx] : d.p.elem[idx];
+    if (P < n && !d.have[P]) {
+        int cc[3];
+        grid_nbrs(d, P, cc, nb, has);
+        trig = early_trigger(d, P, nb, has);
+    }
+    const bool take = trig != INT64_MAX;
+    const unsigned long long b = __ballot(take);
+    if (!b) return;
+    const int lane = threadIdx.x & 63, first = __ffsll((long long)b) - 1;
+    int base = 0;
+    if (lane == first) base = atomicAdd(nt, __popcll(b));
+    base = __shfl(base, first, 64);
+    if (!take) return;
+    const int64_t t = base + __popcll(b & ((1ull << lane) - 1ull));
+    list[t] = (int)P;
+    if constexpr (SNAP) {
+        if (t >= s.cap) return;
+        s.P[t] = (int)P;
+        s.te[t] = d.exit_time[trig];
+        for (int q = 0; q < 7; q++) {
+            const int64_t idx = q < 6 ? nb[q] : P;
+            const bool ok = q == 6 || has[q];
+            for (int c = 0; c < 3; c++) s.X[(q * 3 + c) * s.cap + t] = ok ? d.p.X[c][idx] : 0.0;
+            int left = 0, elem = -1;
+            if (ok) {
+                left = d.p.left[idx];
+                const bool updated = idx < trig && d.advected[idx] && !d.exited[idx];
+                elem = updated ? d.elem_new[idx] : d.p.elem[idx];
+            }
+            s.left[q * s.cap + t] = left;
+            s.elem[q * s.cap + t] = elem;
         }
-        s.left[q * s.cap + t] = left;
-        s.elem[q * s.cap + t] = elem;
     }
 }
 
@@ -1728,26 +1733,45 @@ int launch_ftle_mask(fvc_ftle *f) { return launch_ftle_mask_dev(f->ctx, ftle_dev
 /* early FTLE of one frame for a grid of n points (after its advection, before
  * the position update) */
 int launch_ftle_early(fvc_ctx *c, const FtleDev &d, int64_t n, const DevField &fld, double t1, int itype, double dt) {
-    /* scratch: flags [n], triggered list [n], per-tile offsets and the count
-     * [nb + 1]; the count stays on the device, so nothing here waits */
-    const int nb = (int)((n + CMP_TILE - 1) / CMP_TILE);
-    int *eflags = (int *)scratch(c, sizeof(int) * (2 * (size_t)n + nb + 1));
-    if (!eflags) return FVC_E_NOMEM;
-    int *elist = eflags + n, *offs = elist + n;
-    k_early_flag<<<grid_for(n, BLOCK), BLOCK, 0, c->stream>>>(d, n, eflags);
-    k_cmp_count<<<nb, BLOCK, 0, c->stream>>>(eflags, n, offs);
-    k_scan_small<<<1, 1024, 0, c->stream>>>(offs, nb);
-    k_cmp_scatter<<<nb, BLOCK, 0, c->stream>>>(eflags, n, offs, nullptr, elist);
+    /* scratch: the triggered list [n] and its length, which stays on the
+     * device, so nothing here waits */
+    int *elist = (int *)scratch(c, sizeof(int) * ((size_t)n + 1));
+    if (!elist) return FVC_E_NOMEM;
+    int *nt = elist + n;
+    FVC_HIP(hipMemsetAsync(nt, 0, sizeof(int), c->stream));
+    k_early_list<0><<<grid_for(n, BLOCK), BLOCK, 0, c->stream>>>(d, n, elist, nt, EarlySnap{});
     const unsigned groups = (unsigned)std::min<int64_t>(std::max<int64_t>(n / 8, 1), 16384);
     const unsigned grid = (unsigned)(((int64_t)groups * 8 + BLOCK - 1) / BLOCK);
     if (itype == INT_RK4)
         FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_early,
-                     <<<grid, BLOCK, 0, c->stream>>>(c->mesh, fld, d, elist, offs + nb, (int64_t)-1, t1, itype, dt,
+                     <<<grid, BLOCK, 0, c->stream>>>(c->mesh, fld, d, elist, nt, (int64_t)-1, t1, itype, dt,
                                                      errbuf(c)));
     else
         FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_early_gen,
-                     <<<grid, BLOCK, 0, c->stream>>>(c->mesh, fld, d, elist, offs + nb, t1, itype, dt, errbuf(c)));
+                     <<<grid, BLOCK, 0, c->stream>>>(c->mesh, fld, d, elist, nt, t1, itype, dt, errbuf(c)));
     FVC_HIP(hipGetLastError());
+    return FVC_OK;
+}
+
+/* the slide's two snapshot buffers, at its first RK4 frame */
+static int early_snap_alloc(fvc_ftle *fo) {
+    constexpr int64_t EARLY_CAP = 1 << 18;
+    fvc_ctx *c = fo->ctx;
+    if (fo->snap[0]) return FVC_OK;
+    const int64_t cap = std::min<int64_t>(fo->n, EARLY_CAP);
+    const size_t bytes = early_snap_bytes(cap);
+    if (hipMalloc(&fo->snap[0], bytes) != hipSuccess) fo->snap[0] = nullptr;
+    if (fo->snap[0] && hipMalloc(&fo->snap[1], bytes) != hipSuccess) {
+        hipFree(fo->snap[0]);
+        fo->snap[0] = fo->snap[1] = nullptr;
+    }
+    if (!fo->snap[0]) {
+        (void)hipGetLastError();
+        c->last_error = "early FTLE snapshot alloc";
+        return FVC_E_NOMEM;
+    }
+    fo->snap_cap = cap;
+    c->bytes_used += 2 * (int64_t)bytes;
     return FVC_OK;
 }
 
@@ -1765,44 +1789,19 @@ int launch_ftle_early(fvc_ctx *c, const FtleDev &d, int64_t n, const DevField &f
 int launch_ftle_early_async(fvc_ftle *fo, const FtleDev &d, const DevField &fld, double t1, int itype, double dt) {
     fvc_ctx *c = fo->ctx;
     const int64_t n = fo->n;
-    constexpr int64_t EARLY_CAP = 1 << 18;
-    if (itype != INT_RK4) {
-        int rc = side_join(c);
-        return rc ? rc : launch_ftle_early(c, d, n, fld, t1, itype, dt);
-    }
-    if (!fo->snap[0]) {
-        const int64_t cap = std::min<int64_t>(n, EARLY_CAP);
-        const size_t bytes = early_snap_bytes(cap);
-        if (hipMalloc(&fo->snap[0], bytes) != hipSuccess) fo->snap[0] = nullptr;
-        if (fo->snap[0] && hipMalloc(&fo->snap[1], bytes) != hipSuccess) {
-            hipFree(fo->snap[0]);
-            fo->snap[0] = fo->snap[1] = nullptr;
-        }
-        if (!fo->snap[0]) {
-            (void)hipGetLastError();
-            c->last_error = "early FTLE snapshot alloc";
-            return FVC_E_NOMEM;
-        }
-        fo->snap_cap = cap;
-        c->bytes_used += 2 * (int64_t)bytes;
-    }
     int rc = side_join(c);
     if (rc) return rc;
-    const int nb = (int)((n + CMP_TILE - 1) / CMP_TILE);
-    int *eflags = (int *)scratch(c, sizeof(int) * (2 * (size_t)n + nb + 1));
-    if (!eflags) return FVC_E_NOMEM;
-    int *elist = eflags + n, *offs = elist + n;
-    k_early_flag<<<grid_for(n, BLOCK), BLOCK, 0, c->stream>>>(d, n, eflags);
-    k_cmp_count<<<nb, BLOCK, 0, c->stream>>>(eflags, n, offs);
-    k_scan_small<<<1, 1024, 0, c->stream>>>(offs, nb);
-    k_cmp_scatter<<<nb, BLOCK, 0, c->stream>>>(eflags, n, offs, nullptr, elist);
+    if (itype != INT_RK4) return launch_ftle_early(c, d, n, fld, t1, itype, dt);
+    int *elist = (int *)scratch(c, sizeof(int) * (size_t)n);
+    if (!elist) return FVC_E_NOMEM;
     const EarlySnap sn = early_snap_view(fo->snap[fo->snap_sel], fo->snap_cap);
-    k_early_snap<<<grid_for(fo->snap_cap, BLOCK), BLOCK, 0, c->stream>>>(d, elist, offs + nb, sn);
+    k_early_list<1><<<grid_for(n, BLOCK), BLOCK, 0, c->stream>>>(d, n, elist, sn.nt, sn);
     const unsigned groups = (unsigned)std::min<int64_t>(std::max<int64_t>(n / 8, 1), 16384);
     const unsigned grid = (unsigned)(((int64_t)groups * 8 + BLOCK - 1) / BLOCK);
-    FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_early,
-                 <<<grid, BLOCK, 0, c->stream>>>(c->mesh, fld, d, elist, offs + nb, fo->snap_cap, t1, itype, dt,
-                                                 errbuf(c)));
+    if (n > fo->snap_cap)
+        FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_early,
+                     <<<grid, BLOCK, 0, c->stream>>>(c->mesh, fld, d, elist, sn.nt, fo->snap_cap, t1, itype, dt,
+                                                     errbuf(c)));
     FVC_HIP(hipGetLastError());
     FVC_HIP(hipEventRecord(c->side_ready, c->stream));
     FVC_HIP(hipStreamWaitEvent(c->side, c->side_ready, 0));
@@ -1850,15 +1849,30 @@ int launch_ftle_frame(fvc_ftle *f, int lo, int hi, double tmin, double tmax, dou
     fld.rkf_tol = ip.rkf_accuracy;
     FtleDev d = ftle_dev(f);
     const int itype = ip.int_type == FVC_INT_RK4 ? INT_RK4 : ip.int_type == FVC_INT_RKF ? INT_RKF : INT_EULER;
-    int *flags = (int *)scratch(c, sizeof(int) * (size_t)f->n);
-    if (!flags) return FVC_E_NOMEM;
-    k_ftle_flags<<<grid_for(f->n, BLOCK), BLOCK, 0, c->stream>>>(d, f->n, ip.extrapolate, f->zperm, flags);
-    FVC_HIP(hipGetLastError());
-    /* the counter is cleared before the compaction's count read-back, so the
-     * advection launches right after that synchronisation */
-    FVC_HIP(hipMemsetAsync(c->d_steps, 0, sizeof(unsigned long long), c->stream));
-    int rc = launch_compact(c, flags, f->n, f->active, &f->nactive, f->zperm);
-    if (rc) return rc;
+    int rc;
+    /* The list of points to integrate is built when there is none (a new or
+     * reset slide, another extrapolation flag) and again once more than a
+     * sixteenth of it has left (their lanes idle until then): a build is four
+     * launches and a wait, 35-40 us and more than its idle lanes cost. */
+    if (f->nactive < 0 || f->active_extrap != ip.extrapolate || f->active_gone * 16 > f->nactive) {
+        int *flags = (int *)scratch(c, sizeof(int) * (size_t)f->n);
+        if (!flags) return FVC_E_NOMEM;
+        k_ftle_flags<<<grid_for(f->n, BLOCK), BLOCK, 0, c->stream>>>(d, f->n, ip.extrapolate, f->zperm, flags);
+        FVC_HIP(hipGetLastError());
+        f->nactive = -1;
+        int64_t listed = 0;
+        if ((rc = launch_compact(c, flags, f->n, f->active, &listed, f->zperm))) return rc;
+        f->nactive = listed;
+        f->active_extrap = ip.extrapolate;
+        f->active_gone = 0;
+    }
+    if (f->nactive > 0) {
+        if (itype == INT_RK4 && !ip.extrapolate) {
+            if ((rc = early_snap_alloc(f))) return rc;
+            /* its last early FTLE ran two frames ago; the last frame joined it */
+            d.early_nt = early_snap_view(f->snap[f->snap_sel], f->snap_cap).nt;
+        }
+    }
     if (f->nactive > 0) {
         timing_begin(c);
         if (itype == 1 && !ip.extrapolate)
@@ -1879,7 +1893,8 @@ int launch_ftle_frame(fvc_ftle *f, int lo, int hi, double tmin, double tmax, dou
         if ((rc = launch_ftle_update_all(c, d, f->n, ip.extrapolate))) return rc;
     }
     rc = check_err(c, "fvc_ftle_frame");
-    c->last_steps = (int64_t)c->h_status->steps[0];
+    take_steps(c);
+    f->active_gone = c->last_idle;
     if (f->nactive > 0) timing_collect(c, c->last_steps);
     return rc;
 }

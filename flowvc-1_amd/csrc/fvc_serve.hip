@@ -551,7 +551,7 @@ static SrvDev srv_dev(fvc_server *S, int k, int parity) {
     d.t0 = S->sp.frame_t0;
     d.fdt = S->sp.frame_dt;
     d.dt = S->sp.time_step;
-    d.steps = S->ctx->d_steps;
+    d.steps = S->ctx->d_steps + 2;
     d.err = S->ctx->d_err;
     d.where = S->ctx->d_where;
     return d;
