@@ -1237,22 +1237,25 @@ extern "C" int fvc_locate(fvc_ctx *c, const double *xyz, const int32_t *guess, i
         return FVC_E_INVALID;
     if (c->mesh.mesh_type != 1) return set_err(c, FVC_E_INVALID, "location needs an unstructured mesh");
     if (n == 0) return FVC_OK;
-    double *dx = nullptr;
-    int *dg = nullptr, *dout = nullptr;
-    FVC_HIP(hipMallocAsync((void **)&dx, sizeof(double) * 3 * n, c->stream));
-    FVC_HIP(hipMallocAsync((void **)&dg, sizeof(int) * n, c->stream));
-    FVC_HIP(hipMallocAsync((void **)&dout, sizeof(int) * n, c->stream));
-    FVC_HIP(hipMemcpyAsync(dx, xyz, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream));
-    if (guess) FVC_HIP(hipMemcpyAsync(dg, guess, sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
+    /* points, guesses and results in the context's scratch (an allocation of
+     * its own cost each call 60 us), results out through the pinned staging */
+    const size_t nb = (size_t)n;
+    double *dx = (double *)fvc::scratch(c, 32 * nb);
+    if (!dx) return set_err(c, FVC_E_NOMEM, "location scratch");
+    int *dg = (int *)(dx + 3 * nb), *dout = dg + nb;
+    FVC_HIP(hipMemcpyAsync(dx, xyz, sizeof(double) * 3 * nb, hipMemcpyHostToDevice, c->stream));
+    if (guess) FVC_HIP(hipMemcpyAsync(dg, guess, sizeof(int) * nb, hipMemcpyHostToDevice, c->stream));
     int rc = launch_locate(c, dx, guess ? dg : nullptr, n, mode, dout);
-    if (!rc) {
-        FVC_HIP(hipMemcpyAsync(elem, dout, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
+    if (rc) return rc;
+    const size_t out = sizeof(int) * nb;
+    if (out < STAGE_MIN && c->stage && c->stage_bytes >= out) {
+        FVC_HIP(hipMemcpyAsync(c->stage, dout, out, hipMemcpyDeviceToHost, c->stream));
         FVC_HIP(hipStreamSynchronize(c->stream));
+        host_copy(elem, c->stage, out);
+        return FVC_OK;
     }
-    hipFreeAsync(dx, c->stream);
-    hipFreeAsync(dg, c->stream);
-    hipFreeAsync(dout, c->stream);
-    hipStreamSynchronize(c->stream);
+    rc = copy_to_host(c, elem, dout, out);
+    if (!rc) FVC_HIP(hipStreamSynchronize(c->stream));
     return rc;
 }
 

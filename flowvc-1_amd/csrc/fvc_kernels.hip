@@ -395,10 +395,7 @@ __global__ __launch_bounds__(BLOCK) void k_locate(DevMesh m, const double *__res
             }
         }
     }
-    if (mode == FVC_LOCATE_GLOBAL || (mode == FVC_LOCATE_WALK_GLOBAL && res < 0)) {
-        int second;
-        res = hash_global<DIM>(m, x, y, z, second);
-    }
+    if (mode == FVC_LOCATE_GLOBAL || (mode == FVC_LOCATE_WALK_GLOBAL && res < 0)) res = hash_global<DIM>(m, x, y, z);
     out[i] = res;
 }
 
