@@ -185,10 +185,11 @@ __device__ void batch_particle(const DevMesh &m, const BatchDev &b, int i, int b
 }
 
 /* GEN = 0: RK4 releases only (no multistep state in registers), held to
- * 3 waves/SIMD (at most 168 VGPRs); 1: the other integrators, at 2 waves/SIMD
- * (about 235 VGPRs, where 3 waves spill 70-87 of them). */
+ * 3 waves/SIMD (at most 168 VGPRs); 2: AB2 and AB3 releases in the reduced
+ * precisions, the same; 1: any others among them, at 2 waves/SIMD (about 235
+ * VGPRs, where 3 waves spill 70-87 of them). */
 template <int MODE, int BS, int GEN>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(GEN ? 2 : FVC_HOT_WAVES))) void k_batch(DevMesh m, BatchDev b,
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(GEN == 1 ? 2 : FVC_HOT_WAVES))) void k_batch(DevMesh m, BatchDev b,
                                                                                       int budget) {
     const int lane = threadIdx.x & 63;
     const int home = blockIdx.x % NQ;
@@ -350,6 +351,7 @@ struct fvc_batch {
     int64_t n0;         /* particles in releases */
     int64_t cls_n0[2];  /* class 0: RK4 releases, class 1: the others */
     int nrel;
+    int ab_only; /* class 1 holds AB2 and AB3 releases only */
     double t0, fdt, dt;
     int nslots;
     int64_t max_budget; /* per-particle bound on budget units for the whole run */
@@ -408,9 +410,15 @@ static bool block_ok(int prec, int bs) {
     return bs == 256;
 }
 
+/* FP64 has no AB build (GEN = 2): the general one takes its place */
+template <int MODE, int GEN>
+constexpr int gen_of() {
+    return MODE == P_F64 && GEN == 2 ? 1 : GEN;
+}
+
 template <int MODE, int BS, int GEN>
 static const void *kfun() {
-    return reinterpret_cast<const void *>(&k_batch<MODE, BS, GEN>);
+    return reinterpret_cast<const void *>(&k_batch<MODE, BS, gen_of<MODE, GEN>()>);
 }
 
 template <int GEN>
@@ -436,7 +444,8 @@ static int grid_for_batch(fvc_batch *b, int k, int bs, int waves_per_cu) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0)
         cus = 256;
     int blocks_per_cu = 0;
-    const void *fn = k ? batch_kernel<1>(c->precision, bs) : batch_kernel<0>(c->precision, bs);
+    const void *fn = !k ? batch_kernel<0>(c->precision, bs)
+                        : b->ab_only ? batch_kernel<2>(c->precision, bs) : batch_kernel<1>(c->precision, bs);
     if (waves_per_cu > 0) {
         blocks_per_cu = std::max(1, waves_per_cu / (bs / 64));
     } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks_per_cu, fn, bs, 0) != hipSuccess ||
@@ -449,7 +458,9 @@ static int grid_for_batch(fvc_batch *b, int k, int bs, int waves_per_cu) {
 
 template <int MODE, int BS>
 static void launch_k(fvc_batch *b, int k, int grid, int budget, const BatchDev &d) {
-    if (k)
+    if (k && b->ab_only)
+        k_batch<MODE, BS, gen_of<MODE, 2>()><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget);
+    else if (k)
         k_batch<MODE, BS, 1><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget);
     else
         k_batch<MODE, BS, 0><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget);
@@ -546,6 +557,10 @@ extern "C" int fvc_batch_create(fvc_ctx *c, fvc_particles *p, const fvc_release 
     b->cls_n0[0] = cls_n0[0];
     b->cls_n0[1] = cls_n0[1];
     b->nrel = nrel;
+    b->ab_only = 1;
+    for (int r = 0; r < nrel; r++)
+        if (rel[r].int_type != FVC_INT_RK4 && rel[r].int_type != FVC_INT_AB2 && rel[r].int_type != FVC_INT_AB3)
+            b->ab_only = 0;
     b->t0 = t0;
     b->fdt = fdt;
     b->dt = dt;

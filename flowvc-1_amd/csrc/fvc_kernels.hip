@@ -176,6 +176,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_GEN_W
     advect_body<MODE, DIM, UNS, 1>(m, f, p, index, begin, count, t1, t2, itype, dt, extrap, eb, steps);
 }
 
+/* AB2 and AB3 of the reduced-precision modes on unstructured meshes, without
+ * strain rate, exposure time or extrapolation (k_advect_gen takes the rest):
+ * the state machine, 3 waves per SIMD */
+template <int MODE, int DIM, int UNS>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void k_advect_ab(
+    DevMesh m, DevField f, PtrSet p, const int *__restrict__ index, int64_t begin, int64_t count, double t1, double t2,
+    int itype, double dt, ErrBuf eb, unsigned long long *steps) {
+    if constexpr (UNS && MODE != P_F64)
+        advect_body<MODE, DIM, UNS, 2>(m, f, p, index, begin, count, t1, t2, itype, dt, 0, eb, steps);
+}
+
 /* Each particle over its own segment: tt[2q], tt[2q+1] = t1, t2 of particle
  * begin+q, skipped where t1 is NaN (staggered release, tracers.c:336-397). */
 template <int MODE, int DIM, int UNS, int GEN>
@@ -360,6 +371,12 @@ int launch_advect(fvc_ctx *c, PtrSet p, const int *index, int64_t begin, int64_t
                          <<<grid_for(count, block), block, 0, c->stream>>>(c->mesh, f, p, index, begin, count, t1, t2,
                                                                            ip.int_type, ip.time_step, ip.extrapolate,
                                                                            errbuf(c), c->d_steps));
+        else if ((ip.int_type == FVC_INT_AB2 || ip.int_type == FVC_INT_AB3) && c->mesh.mesh_type == 1 &&
+                 c->precision != FVC_PREC_F64 && !ip.extrapolate && !f.sr_lo && !f.cet_lo)
+            FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_advect_ab,
+                         <<<grid_for(count, block), block, 0, c->stream>>>(c->mesh, f, p, index, begin, count, t1, t2,
+                                                                           ip.int_type, ip.time_step, errbuf(c),
+                                                                           c->d_steps));
         else
             FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_advect_gen,
                          <<<grid_for(count, block), block, 0, c->stream>>>(c->mesh, f, p, index, begin, count, t1, t2,
