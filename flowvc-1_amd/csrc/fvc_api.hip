@@ -500,9 +500,6 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
             return FVC_E_HIP;
         }
     }
-    /* the staging that every output of up to STAGE_MIN bytes goes through, here
-     * and not in the first pass (pinning takes about 0.2 ms) */
-    if (!grow_stage(c, STAGE_MIN)) (void)hipGetLastError();
     if (hipMemset(c->d_status, 0, sizeof(fvc_status)) != hipSuccess) {
         fvc_destroy(c);
         return FVC_E_HIP;
@@ -1248,7 +1245,7 @@ extern "C" int fvc_locate(fvc_ctx *c, const double *xyz, const int32_t *guess, i
     int rc = launch_locate(c, dx, guess ? dg : nullptr, n, mode, dout);
     if (rc) return rc;
     const size_t out = sizeof(int) * nb;
-    if (out < STAGE_MIN && c->stage && c->stage_bytes >= out) {
+    if (out < STAGE_MIN && grow_stage(c, out)) {
         FVC_HIP(hipMemcpyAsync(c->stage, dout, out, hipMemcpyDeviceToHost, c->stream));
         FVC_HIP(hipStreamSynchronize(c->stream));
         host_copy(elem, c->stage, out);

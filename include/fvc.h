@@ -139,9 +139,9 @@ typedef struct fvc_ftle fvc_ftle;
  * (connectivity, adjacency and the 64-byte FP32 frame the reduced-precision
  * walks test against), plus the hash; at most 2^26 elements and 2^27 nodes.
  * Host memory: outputs (fvc_particles_get, fvc_ftle_output, ...) stage
- * through pinned memory that the context holds until fvc_destroy: 4 MB, grown
- * to up to 64 MB by the first larger output, which also takes up to 64 MB of
- * device memory to pack its records in. */
+ * through pinned memory that the context allocates on first use, up to 64 MB,
+ * and holds until fvc_destroy; one over 4 MB also takes up to 64 MB of device
+ * memory to pack its records in. */
 int fvc_create(const fvc_mesh_desc *mesh, const fvc_params *params, fvc_ctx **out);
 /* Frees the context; objects still alive on it are released and detached
  * (see Lifetimes above). */
