@@ -86,8 +86,8 @@ def roofline_valu(kernel, steps_per_launch, avg_ms, bpp, default_workload):
     """Roofline of the dominant RK4 kernel against the nearest ceiling.
     Counter passes on the FP32 pipe workload (profiles/pmc_valu_pipe.md,
     pmc_l2_pipe.md, pmc_traffic_pipe.md, pmc_wait_pipe.md) put VALU issue
-    highest (64-68% busy), L2-to-L1 reads at 28-37% of the L2's bandwidth
-    and HBM at 2-4%; the waves wait on their own gathers more than half of
+    highest (77-80% busy), L2-to-L1 reads at 12-15% of the L2's bandwidth
+    and HBM at 3-5%; the waves wait on their gathers and LDS rows 45-48% of
     their cycles (the limiter, reported beside the roofline).  The bound
     reported is VALU issue: achieved = VALU busy SIMD-cycles per
     particle-step (SQ_ACTIVE_INST_VALU x 4 over the particle-steps of the
@@ -112,7 +112,7 @@ def roofline_valu(kernel, steps_per_launch, avg_ms, bpp, default_workload):
                valu_source="profiles/pmc_valu_pipe.md (SQ_ACTIVE_INST_VALU x 4 per particle-step)")
     wait = profile_figure("pmc_wait_pipe.md", "wave_wait_share", kernel)
     if wait is not None:
-        out.update(limiter="gather latency: the kernel's waves wait on their loads %.0f%% of their cycles "
+        out.update(limiter="VALU issue and latency: the kernel's waves wait on loads and LDS %.0f%% of their cycles "
                            "(SQ_WAIT_ANY / SQ_WAVE_CYCLES, profiles/pmc_wait_pipe.md)" % (100 * wait))
     return out
 
