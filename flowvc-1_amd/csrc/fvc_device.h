@@ -1454,7 +1454,7 @@ __device__ __forceinline__ void vel_from_rows(const float4 *rows, NodeVel<MODE, 
     }
 }
 
-/* AB: Adams-Bashforth of order AB (2, 3; 1: by the release, itype) as
+/* AB: Adams-Bashforth of the order that itype names, as
  * interval_run defines it, bit for bit: a step is the first stage and the
  * locate walk, whose element and coordinates the next first stage takes, with
  * RK4 steps while the history is short or the step clipped.  Its tests at the
@@ -1489,6 +1489,7 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
     const double hmin = 1e-12 * fabs(dt), hfull = sign_of(dt, b - a);
     float f0[3] = {0.f, 0.f, 0.f}; /* AB: the step's first slope */
     bool multi = false;            /* AB: the step is not RK4 */
+    bool late = false;             /* the step's end lies outside the loaded interval */
     const double inv_span = 1.0 / (f.tmax - f.tmin);
     int taken = 0, ret = 1;
     int phase = PH_F0, hops = 0;
@@ -1528,7 +1529,9 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
         tl0 = (float)l0;
         tlh = (float)((is.tc + is.h / 2 - f.tmin) * inv_span); /* lies between l0 and l1 */
         tl1 = (float)l1;
-        if ((l0 > 1 + TINY) || (l0 < 0 - TINY) || (l1 > 1 + TINY) || (l1 < 0 - TINY)) err = E_TLOC;
+        if ((l0 > 1 + TINY) || (l0 < 0 - TINY)) err = E_TLOC;
+        late = (l1 > 1 + TINY) || (l1 < 0 - TINY); /* for the stages past the first, which RK4 steps alone have */
+        if (!AB && late) err = E_TLOC;
         return true;
     };
     const int order = itype == INT_AB2 ? 2 : 3;
@@ -1674,6 +1677,10 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
             const bool micro = fabs(is.h) <= hmin, full = fabs(is.h - hfull) <= 1e-9 * fabs(hfull);
             multi = micro || (full && p.nhist >= order - 1);
             if (!multi) {
+                if (late) {
+                    err = E_TLOC;
+                    break;
+                }
                 anchor();
             } else { /* on to the locate walk, the ring back at the first stage */
                 const int last = q3;

@@ -2,6 +2,7 @@
 element frame and node velocities in LDS rows.  Positions, exits and elements
 against the FP64 oracle at block and wave edges, with steps from a fraction of
 an element to several elements long, forward and backward."""
+import ctypes
 import os
 import sys
 
@@ -100,4 +101,47 @@ def test_adams_bashforth_rows_give_the_straight_walks_bits(dims, precision, inte
         stay = a["LeftDomain"] == 0
         np.testing.assert_array_equal(a["X"][stay], b["X"][stay])
         np.testing.assert_array_equal(a["ElementIndex"][stay], b["ElementIndex"][stay])
+    ctx.close()
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32", "bf16", "f16"])
+@pytest.mark.parametrize("integrator", [fvc.INT_AB2, fvc.INT_AB3])
+def test_adams_bashforth_step_may_end_past_the_loaded_interval(precision, integrator):
+    """A multistep step reads the field at its start only, so the last full
+    step of a call may end past the loaded interval, with the bits of the
+    straight walks (which exposure times take); an RK4 step, the first of a
+    history, may not."""
+    bounds, xyz, conn, adj, sl, seeds = _field(3)
+    ctx = fvc.Context(3, bounds, precision, 2, coords=xyz, conn=conn, adj=adj)
+    for s in range(2):
+        ctx.load_slice(s, 0.02 * s, sl[s])
+    recs = ctx.seed_list(seeds(300))
+    dt = 2.0**-10  # steps end on binary fractions, the last inside at 20 dt = 0.0195
+    end = 20 * dt
+    assert end < 0.02 < end + dt
+    L = fvc.lib()
+    L.fvc_cet_reset.argtypes = [ctypes.c_void_p]
+
+    def advect(p, t1, t2, substeps):
+        ip = fvc.IntParams(integrator, 0, dt, 0, 0, 0, substeps, 0.0, 0.0, 0.0)
+        return L.fvc_advect(ctx.h, p.h, 0, 300, t1, t2, 0, 1, 0.0, 0.02, ctypes.byref(ip))
+
+    assert L.fvc_cet_reset(ctx.h) == 0
+    out = []
+    for substeps in (0, 2):
+        p = fvc.Particles(ctx, 300)
+        p.set(recs)
+        print("ab past the interval %s substeps %d" % (precision, substeps), flush=True)
+        assert advect(p, 0.0, end, substeps) == 0
+        assert advect(p, end, end + dt, substeps) == 0
+        out.append(p.get())
+        p.set(recs)
+        assert advect(p, end, end + dt, substeps) == -5  # FVC_E_TLOC_RANGE
+        p.close()
+    a, b = out
+    stay = a["LeftDomain"] == 0
+    assert stay.sum() > 100
+    np.testing.assert_array_equal(a["LeftDomain"], b["LeftDomain"])
+    np.testing.assert_array_equal(a["X"][stay], b["X"][stay])
+    np.testing.assert_array_equal(a["ElementIndex"][stay], b["ElementIndex"][stay])
     ctx.close()
