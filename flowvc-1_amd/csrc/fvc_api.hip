@@ -81,6 +81,7 @@ static bool grow_stage(fvc_ctx *c, size_t want) {
     c->stage_bytes = 0;
     want = std::max(want, (size_t)1 << 20);
     if (hipHostMalloc((void **)&c->stage, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError(); /* the caller goes on without: no later check is to find this error */
         c->stage = nullptr;
         return false;
     }
@@ -132,7 +133,7 @@ static void host_copy(void *dst, const void *src, size_t bytes) {
  * synchronises the stream before reading them. */
 int copy_to_host(fvc_ctx *c, void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return FVC_OK;
-    if (bytes >= STAGE_MIN && !grow_stage(c, std::min(bytes, STAGE_MAX))) (void)hipGetLastError();
+    if (bytes >= STAGE_MIN) grow_stage(c, std::min(bytes, STAGE_MAX));
     if (bytes < STAGE_MIN || !c->stage) {
         FVC_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
         return FVC_OK;
