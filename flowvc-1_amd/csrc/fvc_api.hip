@@ -67,120 +67,157 @@ int side_sync(fvc_ctx *c) {
     return hipStreamSynchronize(c->side) == hipSuccess ? FVC_OK : FVC_E_HIP;
 }
 
-/* pinned staging memory: copies from STAGE_MIN on go through it, in rounds of
- * at most STAGE_MAX */
-constexpr size_t STAGE_MIN = (size_t)4 << 20, STAGE_MAX = (size_t)64 << 20, CHUNK = (size_t)8 << 20;
+/* Outputs.  Kernels write results, packed as the host wants them, straight
+ * into pinned memory, and host threads copy them out.  Up to IO_BYTES use the
+ * block that holds the status words since fvc_create: nothing is allocated.
+ * More goes in chunks through the slots of a ring, one kernel and event a
+ * chunk; a thread that has emptied a slot sends the slot's next chunk, so the
+ * host's copies (page faults of fresh memory, mostly) overlap the kernels'
+ * writes.  Why kernels and not the copy engine: 256 KB 22 us against 62, 4 MB
+ * 93 against 209 (pageable memory 111-170 and 625-1,113), 64 MB 1.25 ms
+ * against 1.18; and no packed copy on the device.  Why the ring is small and
+ * late: pinning costs 50-90 us for 1 MB and 300-900 us from 2 MB on, so a
+ * context's first output of up to FIRST_MAX goes through the block too, a
+ * ring of RING_MIN is allocated with the next, and one of RING_MAX only for
+ * outputs whose own copy takes longer. */
+constexpr size_t IO_BLOCK = (size_t)256 << 10, IO_BYTES = IO_BLOCK - 256;
+constexpr size_t FIRST_MAX = (size_t)1 << 20, RING_MIN = (size_t)1 << 20, RING_MAX = (size_t)8 << 20;
+constexpr size_t CHUNK = (size_t)1 << 20; /* host bytes a chunk, a quarter of it for outputs of up to 8 MB */
+static_assert(sizeof(fvc_status) <= IO_BLOCK - IO_BYTES, "the status words lie before the small outputs");
 
-/* the pinned staging buffer, at least `want` (<= STAGE_MAX) bytes; false when
- * it cannot be had */
+/* Rings that contexts have given back, for the next that need one: at most
+ * KEEP_RINGS, the largest, and none once no context lives.  A new ring costs
+ * its pinning and, at the host's first reading, a page fault for every 4 KB:
+ * the first 8 MB output of a new context took 1.2 ms more than its second. */
+constexpr size_t KEEP_RINGS = 2;
+struct Ring {
+    char *p;
+    size_t bytes;
+};
+static std::mutex g_ring_mu;
+static std::vector<Ring> g_rings; /* ascending */
+static int g_contexts = 0;
+
+static void keep_ring(Ring r) {
+    {
+        std::lock_guard<std::mutex> lk(g_ring_mu);
+        if (g_contexts > 0) {
+            size_t k = 0; /* ring_contexts has reserved the room */
+            while (k < g_rings.size() && g_rings[k].bytes < r.bytes) k++;
+            g_rings.insert(g_rings.begin() + k, r);
+            if (g_rings.size() <= KEEP_RINGS) return;
+            r = g_rings[0];
+            g_rings.erase(g_rings.begin());
+        }
+    }
+    hipHostFree(r.p);
+}
+
+static void ring_contexts(int change) {
+    std::vector<Ring> drop;
+    {
+        std::lock_guard<std::mutex> lk(g_ring_mu);
+        g_contexts += change;
+        if (g_contexts == 0) drop.swap(g_rings);
+        else g_rings.reserve(KEEP_RINGS + 1);
+    }
+    for (const Ring &r : drop) hipHostFree(r.p);
+}
+
+/* the ring, at least `want` bytes; false when it cannot be had */
 static bool grow_stage(fvc_ctx *c, size_t want) {
-    if (c->stage && c->stage_bytes >= want) return true;
+    if (c->stage_bytes >= want) return true;
     if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
-    if (c->stage) hipHostFree(c->stage);
-    c->stage = nullptr;
-    c->stage_bytes = 0;
-    want = std::max(want, (size_t)1 << 20);
-    if (hipHostMalloc((void **)&c->stage, want, hipHostMallocDefault) != hipSuccess) {
+    Ring got{nullptr, want};
+    {
+        std::lock_guard<std::mutex> lk(g_ring_mu);
+        for (size_t k = 0; k < g_rings.size(); k++)
+            if (g_rings[k].bytes >= want) {
+                got = g_rings[k];
+                g_rings.erase(g_rings.begin() + k);
+                break;
+            }
+    }
+    if (!got.p &&
+        hipHostMalloc((void **)&got.p, want, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError(); /* the caller goes on without: no later check is to find this error */
-        c->stage = nullptr;
         return false;
     }
-    c->stage_bytes = want;
+    if (c->stage) keep_ring({c->stage, c->stage_bytes});
+    c->stage = got.p;
+    c->stage_bytes = got.bytes;
     return true;
 }
 
-/* the device buffer that records are packed in, at least `want` bytes */
-static int grow_pack(fvc_ctx *c, size_t want) {
-    if (c->pack_bytes >= want) return FVC_OK;
-    FVC_HIP(hipStreamSynchronize(c->stream));
-    if (c->pack) hipFree(c->pack);
-    c->pack = nullptr;
-    c->pack_bytes = 0;
-    FVC_HIP(hipMalloc((void **)&c->pack, want));
-    c->pack_bytes = want;
-    return FVC_OK;
-}
-
-/* memcpy over up to 8 host threads, one for each 512 KB */
-static void host_copy(void *dst, const void *src, size_t bytes) {
-    const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    const int nthr = (int)std::min<size_t>({8, std::max(1u, hw / 2), std::max<size_t>(1, bytes >> 19)});
-    auto part = [&](int t) {
-        const size_t lo = (bytes * t / nthr) & ~(size_t)63, hi = t + 1 == nthr ? bytes : (bytes * (t + 1) / nthr) & ~(size_t)63;
-        memcpy((char *)dst + lo, (const char *)src + lo, hi - lo);
+/* n records to the host, `staged` bytes each in pinned memory and `host`
+ * bytes in the caller's: pack(begin, count, to) enqueues the kernel that
+ * writes `count` of them from `begin` on, take(begin, count, from) moves them
+ * to the caller's memory, on one of several threads.  Complete on return. */
+template <class Pack, class Take>
+static int out_chunks(fvc_ctx *c, int64_t n, size_t staged, size_t host, Pack pack, Take take) {
+    const size_t total = host * (size_t)n, once = staged * (size_t)n;
+    /* chunks of up to 1 MB of the host's bytes where there are many, else a
+     * quarter of a small output each, as far as the slots hold them */
+    int slots = total > RING_MAX ? 8 : 4;
+    int64_t per = total > RING_MAX ? (int64_t)(CHUNK / host) : (n + slots - 1) / slots;
+    size_t bytes = staged * (size_t)per * slots > 2 * RING_MIN ? RING_MAX : RING_MIN;
+    if (total <= RING_MAX) bytes = RING_MIN;
+    char *ring;
+    if (once <= IO_BYTES || (!c->stage && !c->staged_once && once <= FIRST_MAX) || !grow_stage(c, bytes)) {
+        slots = once <= IO_BYTES ? 1 : 2; /* through the block */
+        ring = (char *)c->h_status + (IO_BLOCK - IO_BYTES);
+        bytes = IO_BYTES;
+        if (slots == 1) per = n;
+    } else {
+        ring = c->stage;
+    }
+    per = std::min(per, (int64_t)((bytes / slots & ~(size_t)255) / staged));
+    c->staged_once = c->staged_once || slots > 1;
+    const size_t slot_bytes = (staged * (size_t)per + 255) & ~(size_t)255;
+    const int64_t nch = (n + per - 1) / per;
+    slots = (int)std::min<int64_t>(nch, slots);
+    while ((int)c->stage_ev.size() < slots) {
+        hipEvent_t ev;
+        FVC_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming | hipEventReleaseToSystem));
+        c->stage_ev.push_back(ev);
+    }
+    auto send = [&](int64_t q) {
+        pack(q * per, std::min(per, n - q * per), ring + (q % slots) * slot_bytes);
+        return hipGetLastError() == hipSuccess && hipEventRecord(c->stage_ev[q % slots], c->stream) == hipSuccess;
+    };
+    std::atomic<int> failed{0};
+    for (int64_t q = 0; q < slots && !failed; q++)
+        if (!send(q)) failed = 1;
+    /* a thread for each MB from 2 MB on (starting one costs 15-30 us, the copy
+     * of a MB 12 us into warm memory and 215 into fresh); a power of two, so
+     * that the thread that empties a slot waits for the slot's next chunk */
+    const unsigned hw = std::max(2u, std::thread::hardware_concurrency());
+    int nthr = 1;
+    while (2 * nthr <= (int)std::min<unsigned>(8, hw / 2) && 2 * nthr <= slots && ((size_t)nthr << 21) <= total) nthr *= 2;
+    auto worker = [&](int t) {
+        if (t && hipSetDevice(c->device) != hipSuccess) failed = 1;
+        for (int64_t q = t; q < nch && !failed; q += nthr) {
+            if (hipEventSynchronize(c->stage_ev[q % slots]) != hipSuccess) {
+                failed = 1;
+                return;
+            }
+            take(q * per, std::min(per, n - q * per), ring + (q % slots) * slot_bytes);
+            if (q + slots < nch && !send(q + slots)) failed = 1;
+        }
     };
     std::vector<std::thread> pool;
     try {
-        for (int t = 1; t < nthr; t++) pool.emplace_back(part, t);
-    } catch (...) { /* fewer threads: the calling thread copies the rest */
+        for (int t = 1; t < nthr; t++) pool.emplace_back(worker, t);
+    } catch (...) { /* fewer threads: the calling thread does the rest */
     }
     const int started = (int)pool.size() + 1;
-    part(0);
-    for (int t = started; t < nthr; t++) part(t);
+    worker(0);
     for (auto &th : pool) th.join();
-}
-
-/* Device -> host copy of a large block into caller (pageable) memory.  The
- * runtime moves pageable destinations through its own small staging buffer,
- * about 12 GB/s on a 168 MB copy; DMA into pinned memory runs at the link's
- * rate.  So the block goes in chunks into the context's pinned staging
- * buffer (grown to the copy's size, at most STAGE_MAX; larger copies go in
- * rounds), an event after each chunk, and host threads copy each chunk out,
- * each its own stripe, as soon as its event has completed: the host copy
- * overlaps the DMA of the chunks behind it; dst is complete on return.
- * Blocks under STAGE_MIN, or all blocks when the pinned buffer cannot be
- * had, are only enqueued on the stream as a direct copy: the caller
- * synchronises the stream before reading them. */
-int copy_to_host(fvc_ctx *c, void *dst, const void *src, size_t bytes) {
-    if (bytes == 0) return FVC_OK;
-    if (bytes >= STAGE_MIN) grow_stage(c, std::min(bytes, STAGE_MAX));
-    if (bytes < STAGE_MIN || !c->stage) {
-        FVC_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-        return FVC_OK;
-    }
-    const size_t max_chunks = (c->stage_bytes + CHUNK - 1) / CHUNK;
-    while (c->stage_ev.size() < max_chunks) {
-        hipEvent_t ev;
-        FVC_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-        c->stage_ev.push_back(ev);
-    }
-    const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    const int nthr = (int)std::min(8u, std::max(1u, hw / 2));
-    for (size_t done = 0; done < bytes;) {
-        const size_t round = std::min(bytes - done, c->stage_bytes);
-        const size_t nch = (round + CHUNK - 1) / CHUNK;
-        for (size_t k = 0; k < nch; k++) {
-            const size_t off = k * CHUNK, len = std::min(CHUNK, round - off);
-            FVC_HIP(hipMemcpyAsync(c->stage + off, (const char *)src + done + off, len, hipMemcpyDeviceToHost,
-                                   c->stream));
-            FVC_HIP(hipEventRecord(c->stage_ev[k], c->stream));
-        }
-        std::atomic<int> failed{0};
-        auto worker = [&](int t) {
-            for (size_t k = 0; k < nch; k++) {
-                const size_t off = k * CHUNK, len = std::min(CHUNK, round - off);
-                const size_t lo = (len * t / nthr) & ~(size_t)63, hi = t + 1 == nthr ? len : (len * (t + 1) / nthr) & ~(size_t)63;
-                if (hipEventSynchronize(c->stage_ev[k]) != hipSuccess) {
-                    failed = 1;
-                    return;
-                }
-                if (hi > lo) memcpy((char *)dst + done + off + lo, c->stage + off + lo, hi - lo);
-            }
-        };
-        std::vector<std::thread> pool;
-        try {
-            for (int t = 1; t < nthr; t++) pool.emplace_back(worker, t);
-        } catch (...) { /* fewer threads: the calling thread copies the rest */
-        }
-        const int started = (int)pool.size() + 1;
-        worker(0);
-        for (auto &th : pool) th.join();
-        for (int t = started; t < nthr; t++) worker(t);
-        if (failed) {
-            c->last_error = "device to host copy failed";
-            return FVC_E_HIP;
-        }
-        done += round;
+    for (int t = started; t < nthr; t++) worker(t);
+    if (failed) {
+        hipStreamSynchronize(c->stream);
+        c->last_error = "device to host copy failed";
+        return FVC_E_HIP;
     }
     return FVC_OK;
 }
@@ -456,6 +493,7 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= pp->device || pp->device < 0) return FVC_E_NODEVICE;
     if (hipSetDevice(pp->device) != hipSuccess) return FVC_E_NODEVICE;
     fvc_ctx *c = new fvc_ctx();
+    ring_contexts(1);
     c->device = pp->device;
     c->precision = pp->precision;
     c->max_slices = pp->max_slices;
@@ -472,6 +510,7 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
     m.walk_limit = pp->walk_limit > 0 ? pp->walk_limit : (1 << 20);
     int rc = FVC_OK;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
+        ring_contexts(-1);
         delete c;
         return FVC_E_HIP;
     }
@@ -482,7 +521,7 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
     c->d_err = &c->d_status->err;
     c->d_where = &c->d_status->where;
     c->d_steps = c->d_status->steps;
-    if (hipHostMalloc((void **)&c->h_status, sizeof(fvc_status), hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void **)&c->h_status, IO_BLOCK, hipHostMallocCoherent) != hipSuccess) {
         c->h_status = nullptr;
         fvc_destroy(c);
         return FVC_E_NOMEM;
@@ -620,7 +659,6 @@ extern "C" void fvc_destroy(fvc_ctx *c) {
         if (s) hipFree(s);
     if (c->cet_lo) hipFree(c->cet_lo);
     if (c->cet_enc) hipFree(c->cet_enc);
-    if (c->pack) hipFree(c->pack);
     hipFree(c->X64);
     hipFree(c->ER);
     hipFree(c->conn);
@@ -629,7 +667,8 @@ extern "C" void fvc_destroy(fvc_ctx *c) {
     hipFree(c->cell_elems);
     hipFree(c->d_status);
     if (c->h_status) hipHostFree(c->h_status);
-    if (c->stage) hipHostFree(c->stage);
+    if (c->stage) keep_ring({c->stage, c->stage_bytes});
+    ring_contexts(-1);
     for (hipEvent_t ev : c->stage_ev) hipEventDestroy(ev);
     if (c->scratch) hipFree(c->scratch);
     if (c->ev0) hipEventDestroy(c->ev0);
@@ -978,66 +1017,37 @@ __global__ __launch_bounds__(256) void k_pack_points(PackPoints s, int64_t n, do
     out[t] = v;
 }
 
+/* n positions, then, where asked for, the n left flags */
 __global__ __launch_bounds__(256) void k_pack_xyz(const double *__restrict__ x, const double *__restrict__ y,
-                                                  const double *__restrict__ z, int64_t n, double *__restrict__ out) {
+                                                  const double *__restrict__ z, const int *__restrict__ left,
+                                                  int64_t n, double *__restrict__ out) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 3 * n) return;
-    const int64_t i = t / 3;
-    const int a = (int)(t - 3 * i);
-    out[t] = a == 0 ? x[i] : a == 1 ? y[i] : z[i];
-}
-
-/* n records of rec bytes to dst: pack(begin, count, device pointer) enqueues
- * the kernel that writes `count` of them from `begin` on.  Up to STAGE_MIN
- * bytes (latency counts) straight into the pinned buffer, one launch and one
- * wait; more in rounds through a device buffer and copy_to_host.  `more`
- * further bytes follow in the same wait, from `src2` on the device. */
-template <class F>
-static int out_records(fvc_ctx *c, void *dst, int64_t n, size_t rec, F pack, void *dst2 = nullptr,
-                       const void *src2 = nullptr, size_t more = 0) {
-    const size_t total = rec * (size_t)n, at2 = (total + 255) & ~(size_t)255;
-    if (at2 + more <= STAGE_MIN && grow_stage(c, at2 + more)) {
-        pack((int64_t)0, n, c->stage);
-        FVC_HIP(hipGetLastError());
-        if (more) FVC_HIP(hipMemcpyAsync(c->stage + at2, src2, more, hipMemcpyDeviceToHost, c->stream));
-        FVC_HIP(hipStreamSynchronize(c->stream));
-        host_copy(dst, c->stage, total);
-        if (more) memcpy(dst2, c->stage + at2, more);
-        return FVC_OK;
+    if (t < 3 * n) {
+        const int64_t i = t / 3;
+        const int a = (int)(t - 3 * i);
+        out[t] = a == 0 ? x[i] : a == 1 ? y[i] : z[i];
+    } else if (left && t < 4 * n) {
+        reinterpret_cast<int *>(out + 3 * n)[t - 3 * n] = left[t - 3 * n];
     }
-    const int64_t round = std::min<int64_t>(n, (int64_t)(STAGE_MAX / rec));
-    int rc0 = grow_pack(c, rec * (size_t)round);
-    if (rc0) return rc0;
-    for (int64_t b = 0; b < n; b += round) {
-        const int64_t k = std::min(round, n - b);
-        pack(b, k, c->pack);
-        FVC_HIP(hipGetLastError());
-        int rc = copy_to_host(c, (char *)dst + rec * (size_t)b, c->pack, rec * (size_t)k);
-        if (rc) return rc;
-        FVC_HIP(hipStreamSynchronize(c->stream));
-    }
-    if (more) {
-        int rc = copy_to_host(c, dst2, src2, more);
-        if (rc) return rc;
-        FVC_HIP(hipStreamSynchronize(c->stream));
-    }
-    return FVC_OK;
 }
 
 static int out_points(fvc_ctx *c, fvc_point *recs, int64_t n, const PackPoints &src) {
-    return out_records(c, recs, n, sizeof(fvc_point), [&](int64_t b, int64_t k, char *to) {
-        PackPoints s = src;
-        for (int a = 0; a < 3; a++) {
-            if (s.X[a]) s.X[a] += b;
-            if (s.V[a]) s.V[a] += b;
-        }
-        s.lt += b;
-        if (s.scalar) s.scalar += b;
-        if (s.elem) s.elem += b;
-        if (s.aux) s.aux += b;
-        s.left += b;
-        k_pack_points<<<(unsigned)((5 * k + 255) / 256), 256, 0, c->stream>>>(s, k, (double2 *)to);
-    });
+    return out_chunks(
+        c, n, sizeof(fvc_point), sizeof(fvc_point),
+        [&](int64_t b, int64_t k, char *to) {
+            PackPoints s = src;
+            for (int a = 0; a < 3; a++) {
+                if (s.X[a]) s.X[a] += b;
+                if (s.V[a]) s.V[a] += b;
+            }
+            s.lt += b;
+            if (s.scalar) s.scalar += b;
+            if (s.elem) s.elem += b;
+            if (s.aux) s.aux += b;
+            s.left += b;
+            k_pack_points<<<(unsigned)((5 * k + 255) / 256), 256, 0, c->stream>>>(s, k, (double2 *)to);
+        },
+        [&](int64_t b, int64_t k, const char *from) { memcpy(recs + b, from, sizeof(fvc_point) * (size_t)k); });
 }
 
 extern "C" int fvc_particles_get(fvc_particles *p, int64_t begin, fvc_point *recs, int64_t n) {
@@ -1115,13 +1125,18 @@ extern "C" int fvc_particles_get_xyz(fvc_particles *p, int64_t begin, double *xy
     if (!p || !p->ctx || !xyz || begin < 0 || n < 0 || begin + n > p->cap) return FVC_E_INVALID;
     if (n == 0) return FVC_OK;
     fvc_ctx *c = p->ctx;
-    return out_records(
-        c, xyz, n, 3 * sizeof(double),
+    const size_t rec = 3 * sizeof(double) + (left ? sizeof(int) : 0);
+    return out_chunks(
+        c, n, rec, rec,
         [&](int64_t b, int64_t k, char *to) {
-            k_pack_xyz<<<(unsigned)((3 * k + 255) / 256), 256, 0, c->stream>>>(
-                p->X[0] + begin + b, p->X[1] + begin + b, p->X[2] + begin + b, k, (double *)to);
+            k_pack_xyz<<<(unsigned)((4 * k + 255) / 256), 256, 0, c->stream>>>(
+                p->X[0] + begin + b, p->X[1] + begin + b, p->X[2] + begin + b, left ? p->left + begin + b : nullptr, k,
+                (double *)to);
         },
-        left, p->left + begin, left ? sizeof(int) * (size_t)n : 0);
+        [&](int64_t b, int64_t k, const char *from) {
+            memcpy(xyz + 3 * b, from, 3 * sizeof(double) * (size_t)k);
+            if (left) memcpy(left + b, from + 3 * sizeof(double) * (size_t)k, sizeof(int) * (size_t)k);
+        });
 }
 
 /* ------------------------------------------------------------------------ */
@@ -1230,13 +1245,18 @@ extern "C" int fvc_last_step_count(fvc_ctx *c, int64_t *n) {
 /* ------------------------------------------------------------------------ */
 /* location                                                                   */
 /* ------------------------------------------------------------------------ */
+__global__ __launch_bounds__(256) void k_out_ints(const int *__restrict__ src, int64_t n, int *__restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = src[i];
+}
+
 extern "C" int fvc_locate(fvc_ctx *c, const double *xyz, const int32_t *guess, int64_t n, int32_t mode, int32_t *elem) {
     if (!c || !xyz || !elem || n < 0 || mode < 0 || mode > 2 || (mode != FVC_LOCATE_GLOBAL && !guess))
         return FVC_E_INVALID;
     if (c->mesh.mesh_type != 1) return set_err(c, FVC_E_INVALID, "location needs an unstructured mesh");
     if (n == 0) return FVC_OK;
     /* points, guesses and results in the context's scratch (an allocation of
-     * its own cost each call 60 us), results out through the pinned staging */
+     * its own cost each call 60 us) */
     const size_t nb = (size_t)n;
     double *dx = (double *)fvc::scratch(c, 32 * nb);
     if (!dx) return set_err(c, FVC_E_NOMEM, "location scratch");
@@ -1245,16 +1265,12 @@ extern "C" int fvc_locate(fvc_ctx *c, const double *xyz, const int32_t *guess, i
     if (guess) FVC_HIP(hipMemcpyAsync(dg, guess, sizeof(int) * nb, hipMemcpyHostToDevice, c->stream));
     int rc = launch_locate(c, dx, guess ? dg : nullptr, n, mode, dout);
     if (rc) return rc;
-    const size_t out = sizeof(int) * nb;
-    if (out < STAGE_MIN && grow_stage(c, out)) {
-        FVC_HIP(hipMemcpyAsync(c->stage, dout, out, hipMemcpyDeviceToHost, c->stream));
-        FVC_HIP(hipStreamSynchronize(c->stream));
-        host_copy(elem, c->stage, out);
-        return FVC_OK;
-    }
-    rc = copy_to_host(c, elem, dout, out);
-    if (!rc) FVC_HIP(hipStreamSynchronize(c->stream));
-    return rc;
+    return out_chunks(
+        c, n, sizeof(int), sizeof(int),
+        [&](int64_t b, int64_t k, char *to) {
+            k_out_ints<<<(unsigned)((k + 255) / 256), 256, 0, c->stream>>>(dout + b, k, (int *)to);
+        },
+        [&](int64_t b, int64_t k, const char *from) { memcpy(elem + b, from, sizeof(int) * (size_t)k); });
 }
 
 /* ------------------------------------------------------------------------ */
@@ -1311,45 +1327,18 @@ extern "C" int fvc_locate_noalloc(fvc_ctx *c, const double *xyz, const int32_t *
     return FVC_OK;
 }
 
-/* records of located seeds (k_pack_points' layout): positions from the list
- * (z = 0 in 2-D, tracers.c:1033) or the grid */
-struct SeedPack {
-    int chain, dims, mesh_type;
-    const double *xyz;
-    double mn[3], del[3];
-    int res[3];
-    const int *elem, *left;
-    const double *lt;
-};
-
-__global__ __launch_bounds__(256) void k_pack_seeds(SeedPack s, int64_t begin, int64_t n, double2 *__restrict__ out) {
-#pragma clang fp contract(off)
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 5 * n) return;
-    const int64_t i = begin + t / 5;
-    const int part = (int)(t % 5);
-    double2 v = make_double2(0.0, 0.0);
-    if (part < 2) {
-        double X[3];
-        if (s.chain == 0) {
-            for (int a = 0; a < 3; a++) X[a] = s.xyz[3 * i + a];
-            if (s.dims == 2) X[2] = 0.0;
-        } else {
-            const int64_t plane = (int64_t)s.res[0] * s.res[1];
-            const int ii = (int)(i % s.res[0]), jj = (int)((i / s.res[0]) % s.res[1]), kk = (int)(i / plane);
-            X[0] = s.mn[0] + ii * s.del[0];
-            X[1] = s.mn[1] + jj * s.del[1];
-            X[2] = s.mn[2] + kk * s.del[2];
-        }
-        v = part == 0 ? make_double2(X[0], X[1]) : make_double2(X[2], 0.0);
-    } else if (part == 3) {
-        const int e = s.elem[i], l = s.left[i];
-        v = make_double2(__hiloint2double(s.chain == 0 && !l ? e : 0, s.mesh_type == 1 ? e : 0), __hiloint2double(0, l));
-    } else if (part == 4) {
-        v.x = s.lt[i];
-    }
-    out[t] = v;
+/* what the host does not know of a located seed: element, left flag, time */
+__global__ __launch_bounds__(256) void k_pack_seeds(const int *__restrict__ elem, const int *__restrict__ left,
+                                                    const double *__restrict__ lt, int64_t n,
+                                                    double2 *__restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = make_double2(__hiloint2double(left[i], elem[i]), lt[i]);
 }
+
+struct SeedOut {
+    int elem, left;
+    double lt;
+};
 
 static int seed_common(fvc_ctx *c, int chain, const double *xyz, int64_t n, const double mn[3], const double del[3],
                        const int32_t res[3], int lsc, fvc_point *out) {
@@ -1365,15 +1354,48 @@ static int seed_common(fvc_ctx *c, int chain, const double *xyz, int64_t n, cons
     FVC_HIP(hipMallocAsync((void **)&dl, sizeof(int) * n, c->stream));
     int rc = launch_seed_chain(c, chain, n, dx, mn, del, res, lsc, de, dl, dlt);
     if (!rc) {
-        SeedPack s{chain, c->mesh.dims, c->mesh.mesh_type, dx, {0, 0, 0}, {0, 0, 0}, {1, 1, 1}, de, dl, dlt};
-        for (int a = 0; a < 3 && chain != 0; a++) {
-            s.mn[a] = mn[a];
-            s.del[a] = del[a];
-            s.res[a] = res[a];
-        }
-        rc = out_records(c, out, n, sizeof(fvc_point), [&](int64_t b, int64_t k, char *to) {
-            k_pack_seeds<<<(unsigned)((5 * k + 255) / 256), 256, 0, c->stream>>>(s, b, k, (double2 *)to);
-        });
+        const int dims = c->mesh.dims, mesh_type = c->mesh.mesh_type;
+        rc = out_chunks(
+            c, n, sizeof(SeedOut), sizeof(fvc_point),
+            [&](int64_t b, int64_t k, char *to) {
+                k_pack_seeds<<<(unsigned)((k + 255) / 256), 256, 0, c->stream>>>(de + b, dl + b, dlt + b, k,
+                                                                                (double2 *)to);
+            },
+            [&](int64_t b, int64_t k, const char *from) {
+#pragma clang fp contract(off)
+                const SeedOut *s = (const SeedOut *)from;
+                int ii = 0, jj = 0, kk = 0;
+                if (chain != 0) {
+                    ii = (int)(b % res[0]);
+                    jj = (int)((b / res[0]) % res[1]);
+                    kk = (int)(b / ((int64_t)res[0] * res[1]));
+                }
+                for (int64_t q = 0; q < k; q++) {
+                    fvc_point r{};
+                    if (chain == 0) { /* z = 0 in 2-D (tracers.c:1033) */
+                        const double *x = xyz + 3 * (b + q);
+                        r.X[0] = x[0];
+                        r.X[1] = x[1];
+                        r.X[2] = dims == 2 ? 0.0 : x[2];
+                    } else {
+                        r.X[0] = mn[0] + ii * del[0];
+                        r.X[1] = mn[1] + jj * del[1];
+                        r.X[2] = mn[2] + kk * del[2];
+                        if (++ii == res[0]) {
+                            ii = 0;
+                            if (++jj == res[1]) {
+                                jj = 0;
+                                kk++;
+                            }
+                        }
+                    }
+                    r.ElementIndex = mesh_type == 1 ? s[q].elem : 0;
+                    r.AuxElementIndex = chain == 0 && !s[q].left ? s[q].elem : 0;
+                    r.LeftDomain = s[q].left;
+                    r.LeftDomainTime = s[q].lt;
+                    out[b + q] = r;
+                }
+            });
     }
     if (dx) hipFreeAsync(dx, c->stream);
     hipFreeAsync(dlt, c->stream);
@@ -1681,35 +1703,19 @@ __global__ void k_ftle_kji(const double *__restrict__ wt, const double *__restri
     out[n + t] = wot[P];
 }
 
-/* FTLE values of a grid to host memory in the file order of ftle.c:1302-1315:
- * as out_records, but in two blocks */
+/* FTLE values of a grid to host memory in the file order of ftle.c:1302-1315 */
 int fvc::copy_ftle_kji(fvc_ctx *c, const double *d_wt, const double *d_wot, const int32_t res[3], double *wt,
                        double *wot) {
-    const int64_t n = (int64_t)res[0] * res[1] * res[2];
-    const size_t rec = 2 * sizeof(double);
-    auto pack = [&](int64_t b, int64_t k, void *to) {
-        k_ftle_kji<<<(unsigned)((k + 255) / 256), 256, 0, c->stream>>>(d_wt, d_wot, res[0], res[1], res[2], b, k,
-                                                                       (double *)to);
-    };
-    if (rec * (size_t)n <= STAGE_MIN && grow_stage(c, rec * (size_t)n)) {
-        pack(0, n, c->stage);
-        FVC_HIP(hipGetLastError());
-        FVC_HIP(hipStreamSynchronize(c->stream));
-        if (wt) host_copy(wt, c->stage, sizeof(double) * (size_t)n);
-        if (wot) host_copy(wot, (double *)c->stage + n, sizeof(double) * (size_t)n);
-        return FVC_OK;
-    }
-    const int64_t round = std::min<int64_t>(n, (int64_t)(STAGE_MAX / rec));
-    int rc = grow_pack(c, rec * (size_t)round);
-    for (int64_t b = 0; b < n && !rc; b += round) {
-        const int64_t k = std::min(round, n - b);
-        pack(b, k, c->pack);
-        FVC_HIP(hipGetLastError());
-        if (wt) rc = copy_to_host(c, wt + b, c->pack, sizeof(double) * (size_t)k);
-        if (!rc && wot) rc = copy_to_host(c, wot + b, (double *)c->pack + k, sizeof(double) * (size_t)k);
-        FVC_HIP(hipStreamSynchronize(c->stream));
-    }
-    return rc;
+    return out_chunks(
+        c, (int64_t)res[0] * res[1] * res[2], 2 * sizeof(double), 2 * sizeof(double),
+        [&](int64_t b, int64_t k, char *to) {
+            k_ftle_kji<<<(unsigned)((k + 255) / 256), 256, 0, c->stream>>>(d_wt, d_wot, res[0], res[1], res[2], b, k,
+                                                                           (double *)to);
+        },
+        [&](int64_t b, int64_t k, const char *from) {
+            if (wt) memcpy(wt + b, from, sizeof(double) * (size_t)k);
+            if (wot) memcpy(wot + b, from + sizeof(double) * (size_t)k, sizeof(double) * (size_t)k);
+        });
 }
 
 extern "C" int fvc_ftle_output(fvc_ftle *f, double int_t, double *wt, double *wot) {

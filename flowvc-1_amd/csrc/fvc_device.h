@@ -1489,7 +1489,6 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
     const double hmin = 1e-12 * fabs(dt), hfull = sign_of(dt, b - a);
     float f0[3] = {0.f, 0.f, 0.f}; /* AB: the step's first slope */
     bool multi = false;            /* AB: the step is not RK4 */
-    bool late = false;             /* the step's end lies outside the loaded interval */
     const double inv_span = 1.0 / (f.tmax - f.tmin);
     int taken = 0, ret = 1;
     int phase = PH_F0, hops = 0;
@@ -1530,8 +1529,8 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
         tlh = (float)((is.tc + is.h / 2 - f.tmin) * inv_span); /* lies between l0 and l1 */
         tl1 = (float)l1;
         if ((l0 > 1 + TINY) || (l0 < 0 - TINY)) err = E_TLOC;
-        late = (l1 > 1 + TINY) || (l1 < 0 - TINY); /* for the stages past the first, which RK4 steps alone have */
-        if (!AB && late) err = E_TLOC;
+        /* only RK4 steps read the field at their end: AB tests l1 where it knows */
+        if (!AB && ((l1 > 1 + TINY) || (l1 < 0 - TINY))) err = E_TLOC;
         return true;
     };
     const int order = itype == INT_AB2 ? 2 : 3;
@@ -1677,7 +1676,8 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
             const bool micro = fabs(is.h) <= hmin, full = fabs(is.h - hfull) <= 1e-9 * fabs(hfull);
             multi = micro || (full && p.nhist >= order - 1);
             if (!multi) {
-                if (late) {
+                const double l1 = (is.tc + is.h - f.tmin) * inv_span;
+                if ((l1 > 1 + TINY) || (l1 < 0 - TINY)) {
                     err = E_TLOC;
                     break;
                 }

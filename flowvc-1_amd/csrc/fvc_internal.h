@@ -63,14 +63,12 @@ struct fvc_ctx {
     /* scratch (grown on demand) */
     void *scratch;
     size_t scratch_bytes;
-    /* pinned staging of large device -> host copies (copy_to_host), grown on
-     * demand, with one event per chunk */
+    /* pinned ring of outputs (out_chunks), at most 8 MB, with one event per
+     * slot; small outputs go through the pinned block that h_status begins,
+     * and so does the first one that is not (staged_once) */
     char *stage;
     size_t stage_bytes;
-    /* device buffer in which kernels pack records on their way out, grown on
-     * demand to at most OUT_ROUND bytes */
-    char *pack;
-    size_t pack_bytes;
+    bool staged_once;
     std::vector<hipEvent_t> stage_ev;
     /* side stream: an FTLE slide frame's early FTLE (from a snapshot of its
      * stencils) runs there beside the next frame's advection; side_done
@@ -233,7 +231,6 @@ inline void take_steps(fvc_ctx *c) {
 /* order the main stream after the side stream's last launch / wait for it on the host */
 int side_join(fvc_ctx *c);
 int side_sync(fvc_ctx *c);
-int copy_to_host(fvc_ctx *c, void *dst, const void *src, size_t bytes);
 /* release an object's device memory and detach it from its context (the
  * handle stays valid for its *_destroy call only); no-ops when detached */
 void particles_release(fvc_particles *p);

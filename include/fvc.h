@@ -138,10 +138,10 @@ typedef struct fvc_ftle fvc_ftle;
  * Device memory of an unstructured mesh: 32 B per node, 96 B per element
  * (connectivity, adjacency and the 64-byte FP32 frame the reduced-precision
  * walks test against), plus the hash; at most 2^26 elements and 2^27 nodes.
- * Host memory: outputs (fvc_particles_get, fvc_ftle_output, ...) stage
- * through pinned memory that the context allocates on first use, up to 64 MB,
- * and holds until fvc_destroy; one over 4 MB also takes up to 64 MB of device
- * memory to pack its records in. */
+ * Host memory: 256 KB of pinned memory; outputs over that (fvc_particles_get,
+ * fvc_ftle_output, ...) stage through up to 8 MB more, allocated when first
+ * needed and held until fvc_destroy, or through the 256 KB where it cannot be
+ * had. */
 int fvc_create(const fvc_mesh_desc *mesh, const fvc_params *params, fvc_ctx **out);
 /* Frees the context; objects still alive on it are released and detached
  * (see Lifetimes above). */

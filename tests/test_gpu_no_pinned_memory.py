@@ -1,6 +1,6 @@
 """Outputs where pinned host memory cannot be had: the same bytes as with it.
 A process of its own loads a stand-in for hipHostMalloc that refuses blocks
-over 64 KB before the library, and prints a digest of every kind of output."""
+over 256 KB before the library, and prints a digest of every kind of output."""
 import os
 import subprocess
 import sys
