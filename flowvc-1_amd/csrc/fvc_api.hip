@@ -1255,22 +1255,35 @@ extern "C" int fvc_locate(fvc_ctx *c, const double *xyz, const int32_t *guess, i
         return FVC_E_INVALID;
     if (c->mesh.mesh_type != 1) return set_err(c, FVC_E_INVALID, "location needs an unstructured mesh");
     if (n == 0) return FVC_OK;
-    /* points, guesses and results in the context's scratch (an allocation of
-     * its own cost each call 60 us) */
+    /* points, guesses and results (32 B a point) in the context's scratch up
+     * to LOCATE_KEPT points, where an allocation of its own would cost each
+     * call 60 us; more only for the call */
+    constexpr int64_t LOCATE_KEPT = 1 << 20;
     const size_t nb = (size_t)n;
-    double *dx = (double *)fvc::scratch(c, 32 * nb);
-    if (!dx) return set_err(c, FVC_E_NOMEM, "location scratch");
+    void *own = nullptr, *base;
+    if (n <= LOCATE_KEPT) base = fvc::scratch(c, 32 * nb);
+    else base = hipMallocAsync(&own, 32 * nb, c->stream) == hipSuccess ? own : nullptr;
+    if (!base) {
+        (void)hipGetLastError();
+        return set_err(c, FVC_E_NOMEM, "location scratch");
+    }
+    double *dx = (double *)base;
     int *dg = (int *)(dx + 3 * nb), *dout = dg + nb;
-    FVC_HIP(hipMemcpyAsync(dx, xyz, sizeof(double) * 3 * nb, hipMemcpyHostToDevice, c->stream));
-    if (guess) FVC_HIP(hipMemcpyAsync(dg, guess, sizeof(int) * nb, hipMemcpyHostToDevice, c->stream));
-    int rc = launch_locate(c, dx, guess ? dg : nullptr, n, mode, dout);
-    if (rc) return rc;
-    return out_chunks(
-        c, n, sizeof(int), sizeof(int),
-        [&](int64_t b, int64_t k, char *to) {
-            k_out_ints<<<(unsigned)((k + 255) / 256), 256, 0, c->stream>>>(dout + b, k, (int *)to);
-        },
-        [&](int64_t b, int64_t k, const char *from) { memcpy(elem + b, from, sizeof(int) * (size_t)k); });
+    int rc = FVC_OK;
+    if (hipMemcpyAsync(dx, xyz, sizeof(double) * 3 * nb, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+        (guess && hipMemcpyAsync(dg, guess, sizeof(int) * nb, hipMemcpyHostToDevice, c->stream) != hipSuccess))
+        rc = set_err(c, FVC_E_HIP, "location upload");
+    if (!rc) rc = launch_locate(c, dx, guess ? dg : nullptr, n, mode, dout);
+    if (!rc)
+        rc = out_chunks(
+            c, n, sizeof(int), sizeof(int),
+            [&](int64_t b, int64_t k, char *to) {
+                k_out_ints<<<(unsigned)((k + 255) / 256), 256, 0, c->stream>>>(dout + b, k, (int *)to);
+            },
+            [&](int64_t b, int64_t k, const char *from) { memcpy(elem + b, from, sizeof(int) * (size_t)k); });
+    if (own) hipFreeAsync(own, c->stream);
+    if (own || rc) hipStreamSynchronize(c->stream); /* the caller's arrays are no longer read */
+    return rc;
 }
 
 /* ------------------------------------------------------------------------ */

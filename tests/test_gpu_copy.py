@@ -1,8 +1,8 @@
-"""Large device -> host copies (fvc_particles_get, fvc_ftle_output) travel in
-8 MB chunks through a pinned staging buffer of the context (at most 64 MB, so
-larger arrays go in rounds), host threads copying each chunk out in stripes
-while the next chunks' DMA runs; blocks under 4 MB are copied directly.
-Whatever the path, the host must receive the device's bytes exactly."""
+"""Outputs (fvc_particles_get, fvc_ftle_output, ...) are written by kernels
+into pinned memory: up to 256 KB in one piece, larger ones in chunks through a
+ring of 1 MB (8 MB for outputs over 8 MB), host threads emptying its slots
+while the next chunks are written.  Whatever the path, the host must receive
+the device's bytes exactly."""
 import numpy as np
 import pytest
 
@@ -30,9 +30,9 @@ def _same_bytes(a, b):
 
 
 def test_particle_records_round_trip_through_staged_copies():
-    """9M records: each FP64 array is 72 MB (two rounds of the staging
-    buffer, nine chunks, the last one partial), each int32 array 36 MB; then
-    an unaligned sub-range, and a small range that takes the direct copy."""
+    """9M records, 720 MB (687 chunks through the eight slots of the large
+    ring, the last one partial); then an unaligned sub-range, and a small range
+    that goes in one piece."""
     n = 9_000_000
     ctx = fvc.Context(2, [0.0, 2.0, 0.0, 1.0, 0.0, 0.0], "f64", 2, cart_min=[0, 0, 0], cart_max=[2, 1, 0],
                       cart_res=[16, 8, 1])
@@ -49,8 +49,8 @@ def test_particle_records_round_trip_through_staged_copies():
 
 
 def test_large_ftle_output_equals_a_narrow_grid_of_the_same_spacing():
-    """Double-gyre FTLE on a 1101 x 1001 grid (8.8 MB per field: staged) and
-    on its first 101 columns as a grid of their own (0.8 MB: direct copy),
+    """Double-gyre FTLE on a 1101 x 1001 grid (17.6 MB: the large ring) and
+    on its first 101 columns as a grid of their own (1.6 MB: the small one),
     both with spacing 2^-9 so that every grid point is the same double.
     Away from the narrow grid's last column, each point has the same stencil
     in both grids, so both fields agree bit for bit there; wot = wt * T with
@@ -79,9 +79,11 @@ def test_large_ftle_output_equals_a_narrow_grid_of_the_same_spacing():
     ctx.close()
 
 
-# 80-byte records: 52,428 fill the 4 MB that go out in one wait, 838,860 one
-# round of the packing buffer; 24-byte positions: 174,762 and 2,796,202
-@pytest.mark.parametrize("n", [5, 63, 52428, 52429, 174763, 838860, 838861, 1700001])
+# 80-byte records: 3,273 fill the 256 KB that go out in one piece, 13,104 the
+# small ring, 104,857 is the last count of the small ring, 104,960 fill the
+# large one; 28-byte positions with flags: 9,353, 37,449, 299,593 and 299,648
+@pytest.mark.parametrize("n", [5, 63, 3273, 3274, 9353, 9354, 13104, 13105, 37449, 52428, 52429, 104857, 104858, 104961,
+                               174763, 299593, 299594, 299649, 838860, 838861, 1700001])
 def test_packed_records_and_positions_at_round_edges(n):
     ctx = fvc.Context(2, [0.0, 1.0, 0.0, 1.0, 0.0, 0.0], "f64", 2, cart_min=[0.0] * 3, cart_max=[1.0, 1.0, 0.0],
                       cart_res=[4, 4, 1])
@@ -95,4 +97,22 @@ def test_packed_records_and_positions_at_round_edges(n):
     np.testing.assert_array_equal(left, recs["LeftDomain"])
     q.copy_from(p, n, begin=1, src_begin=2)
     assert _same_bytes(q.get(n, begin=1), recs)
+    ctx.close()
+
+
+def test_a_large_location_gives_its_memory_back():
+    """32 bytes a point are held during the call; 192 MB of them afterwards
+    would be missing to later slices and particle sets."""
+    t = host.pipe(6, 6, 10, 1.0, 10.0)
+    xyz, conn, adj = host.tube_mesh(t)
+    ctx = fvc.Context(3, [-1.0, 1.0, -1.0, 1.0, 0.0, 10.0], "f32", 2, coords=xyz, conn=conn, adj=adj)
+    few = host.tube_seeds(t, 1000, 0.0, 10.0, 3)
+    el = ctx.locate(few, None, fvc.LOCATE_GLOBAL)
+    before = ctx.memory()[1]
+    n = 6_000_000
+    print("locate %d points" % n, flush=True)
+    got = ctx.locate(np.resize(few, (n, 3)), None, fvc.LOCATE_GLOBAL)
+    np.testing.assert_array_equal(got, np.resize(el, n))
+    np.testing.assert_array_equal(ctx.locate(np.resize(few, (n, 3)), got, fvc.LOCATE_WALK), got)
+    assert before - ctx.memory()[1] < 64 << 20
     ctx.close()
