@@ -11,6 +11,7 @@
  * Particles are SoA (X,Y,Z,V*,elem,left,left_time,...) for coalesced state I/O.
  */
 #include <hip/hip_runtime.h>
+#include <float.h>
 #include <math.h>
 #include <string.h>
 
@@ -564,7 +565,10 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
             m.cdel[2] = 0;
             m.cres[2] = 1;
         }
-        for (int a = 0; a < 3; a++) m.cinv[a] = fvc_near_inverse(m.cdel[a]);
+        for (int a = 0; a < 3; a++) {
+            m.cinv[a] = fvc_near_inverse(m.cdel[a]);
+            m.cfar[a] = std::min(2.0 * m.cdel[a] * m.cres[a], DBL_MAX);
+        }
         c->nvel = (int64_t)m.cres[0] * m.cres[1] * m.cres[2];
         /* strain-rate cells (strainrate.c:86-91): kmax = 1 in 2-D or for a single z layer */
         c->nsr = (int64_t)(m.cres[0] - 1) * (m.cres[1] - 1) * ((md->dims == 2 || m.cres[2] == 1) ? 1 : m.cres[2] - 1);

@@ -54,6 +54,7 @@ struct DevMesh {
     /* Cartesian velocity grid */
     double cmin[3], cdel[3];
     double cinv[3]; /* 1 / cdel rounded to nearest, 0 where div_near does not apply */
+    double cfar[3]; /* twice the grid's extent: what lies as far from cmin is outside, nearer quotients are finite */
     int cres[3];
     /* unstructured */
     const double4 *__restrict__ X64;
@@ -854,7 +855,7 @@ __device__ __forceinline__ bool cart_cell(const DevMesh &m, const double X[3], i
         for (int a = 0; a < DIM; a++) q[a] = d[a] / m.cdel[a];
     for (int a = 0; a < DIM; a++) {
         const double top = (double)(m.cres[a] - 1);
-        in = in && !(q[a] < 0.0) && !(q[a] > top) && !(fabs(d[a]) >= 1e280);
+        in = in && !(q[a] < 0.0) && !(q[a] > top) && !(fabs(d[a]) >= m.cfar[a]);
         const double fl = floor(q[a]);
         r[a] = d[a] - fl * m.cdel[a];
         cell[a] = (int)fl;

@@ -85,6 +85,20 @@ def test_f64_bit_exact(dims, res, what, n):
             np.testing.assert_array_equal(got[k][fin], ref[k][fin])
 
 
+@pytest.mark.parametrize("dims,res", [(2, [37, 18, 1]), (3, [19, 14, 23])])
+@pytest.mark.parametrize("precision", ["f64", "f32", "bf16", "f16"])
+def test_points_too_far_for_a_finite_quotient_are_outside(dims, res, precision):
+    """(X - min) / del overflows for these points on cells of 1e-92"""
+    size = 1e-90
+    recs = _points(dims, res, size, 300, 8)
+    recs["X"][:40, 0] = np.resize([1e250, -1e250, 1e279, -1e270, 1e300, -1e308, np.inf, -np.inf], 40)
+    recs["X"][40:80, 1] = np.resize([1e250, -1e250, 1e279, -1e270, 1e300, -1e308, np.inf, -np.inf], 40)
+    got, ref = _both(dims, res, size, _grid(dims, res, size), recs, precision, 0.01, 0.0, 0.05)
+    assert (ref["LeftDomain"][:80] != 0).all()
+    for k in ("X", "LeftDomain", "LeftDomainTime"):
+        np.testing.assert_array_equal(got[k][:80], ref[k][:80])
+
+
 # Against FP64: a stage velocity's relative rounding (20 roundings in FP32,
 # half an ulp of the largest value in 16 bits) over T = 0.31 with |u| < 1.1 and
 # gradients up to G = 5, and the FP32 local coordinates' 2^-24.
