@@ -18,7 +18,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdio>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -757,6 +759,26 @@ static inline uint16_t to_f16(float v) {
     return r;
 }
 
+/* FP64 nodes of a slice as the kernels read them, with VALS_* from the sums
+ * of the magnitudes: one that is not finite counts as an infinity, which is as
+ * good (the general path gives the same values).  Twelve sums side by side,
+ * for the vector units. */
+static int slice_nodes(const double *u, int64_t n, double4 *h) {
+    double sum[12] = {};
+    auto node = [&](int64_t i, double *s) {
+        const double *v = u + 3 * i;
+        h[i] = make_double4(v[0], v[1], v[2], 0.0);
+        for (int k = 0; k < 3; k++) s[k] += fabs(v[k]);
+    };
+    int64_t i = 0;
+    for (; i + 4 <= n; i += 4)
+        for (int q = 0; q < 4; q++) node(i + q, sum + 3 * q);
+    for (; i < n; i++) node(i, sum);
+    double all = 0.0;
+    for (double v : sum) all += v;
+    return (all < INFINITY ? 0 : VALS_INF) | (sum[2] + sum[5] + sum[8] + sum[11] == 0.0 ? 0 : VALS_Z);
+}
+
 extern "C" int fvc_load_slice(fvc_ctx *c, int32_t slot, double timestamp, const double *uvw, int64_t n) {
     if (!c || !uvw || slot < 0 || slot >= c->max_slices) return FVC_E_INVALID;
     if (n != c->nvel) return set_err(c, FVC_E_INVALID, "slice length differs from the node count");
@@ -767,20 +789,17 @@ extern "C" int fvc_load_slice(fvc_ctx *c, int32_t slot, double timestamp, const 
         c->bytes_used += (int64_t)(c->vel_stride * (size_t)n);
         c->slices[slot] = p;
     }
-    std::vector<unsigned char> host(c->vel_stride * (size_t)n);
+    const std::unique_ptr<unsigned char[]> host(new (std::nothrow) unsigned char[c->vel_stride * (size_t)n]);
+    if (!host) return set_err(c, FVC_E_NOMEM, "slice conversion");
     float scale = 1.0f;
     int vals = VALS_INF | VALS_Z;
     if (c->precision == FVC_PREC_F64) {
-        double4 *h = (double4 *)host.data();
-        bool inf = false, z = false;
-        for (int64_t i = 0; i < n; i++) {
-            h[i] = make_double4(uvw[3 * i], uvw[3 * i + 1], uvw[3 * i + 2], 0.0);
-            inf = inf | (fabs(h[i].x) == INFINITY) | (fabs(h[i].y) == INFINITY) | (fabs(h[i].z) == INFINITY);
-            z = z | (h[i].z != 0.0);
-        }
-        vals = (inf ? VALS_INF : 0) | (z ? VALS_Z : 0);
+        double4 *h = (double4 *)host.get();
+        if (c->mesh.mesh_type == 0 && c->mesh.dims == 2) vals = slice_nodes(uvw, n, h); /* only their kernels ask */
+        else
+            for (int64_t i = 0; i < n; i++) h[i] = make_double4(uvw[3 * i], uvw[3 * i + 1], uvw[3 * i + 2], 0.0);
     } else if (c->precision == FVC_PREC_F32) {
-        float4 *h = (float4 *)host.data();
+        float4 *h = (float4 *)host.get();
         for (int64_t i = 0; i < n; i++)
             h[i] = make_float4((float)uvw[3 * i], (float)uvw[3 * i + 1], (float)uvw[3 * i + 2], 0.0f);
     } else {
@@ -788,14 +807,14 @@ extern "C" int fvc_load_slice(fvc_ctx *c, int32_t slot, double timestamp, const 
         for (int64_t i = 0; i < 3 * n; i++) mx = std::max(mx, fabs(uvw[i]));
         scale = mx > 0.0 ? (float)mx : 1.0f;
         const double inv = 1.0 / (double)scale;
-        uint16_t *h = (uint16_t *)host.data();
+        uint16_t *h = (uint16_t *)host.get();
         for (int64_t i = 0; i < n; i++)
             for (int q = 0; q < 4; q++) {
                 float v = q < 3 ? (float)(uvw[3 * i + q] * inv) : 0.0f;
                 h[4 * i + q] = c->precision == FVC_PREC_BF16 ? to_bf16(v) : to_f16(v);
             }
     }
-    if (hipMemcpyAsync(c->slices[slot], host.data(), host.size(), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+    if (hipMemcpyAsync(c->slices[slot], host.get(), c->vel_stride * (size_t)n, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return set_err(c, FVC_E_HIP, "slice upload");
     c->slice_scale[slot] = scale;
