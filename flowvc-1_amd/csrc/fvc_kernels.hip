@@ -302,7 +302,7 @@ __global__ __launch_bounds__(BLOCK) void k_advect_times_rk4(DevMesh m, DevField 
                                                            int64_t count, const double *__restrict__ tt, int itype,
                                                            double dt, int extrap, ErrBuf eb, unsigned long long *steps);
 template <int MODE, int DIM, int UNS>
-__global__ __launch_bounds__(BLOCK) void k_advect_times_gen(DevMesh m, DevField f, PtrSet p, int64_t begin,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_GEN_WAVES(MODE)))) void k_advect_times_gen(DevMesh m, DevField f, PtrSet p, int64_t begin,
                                                            int64_t count, const double *__restrict__ tt, int itype,
                                                            double dt, int extrap, ErrBuf eb, unsigned long long *steps);
 
