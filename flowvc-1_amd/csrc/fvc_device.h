@@ -1040,10 +1040,20 @@ __device__ __forceinline__ void cart_velocity_f32(const DevMesh &m, const DevFie
         C lo, hi;
         lo.at(m, f.lo, c0);
         hi.at(m, f.hi, c0);
-        for (int q = 0; q < R::NQ; q++) {
-            cart_words<MODE, DIM>(lo.corner(q * C::STEP), w + 2 * R::W * q);
-            cart_words<MODE, DIM>(hi.corner(q * C::STEP), w + 2 * R::W * q + R::W);
-        }
+        /* Corner x + 1 right after corner x, one line apart at most: between
+         * them the other rows' lines, 64 each, would push theirs out of the
+         * L1 (2-D, 150,000 random points: L1 misses 5.3e7 against 3.1e7 a
+         * launch). */
+        for (int q = 0; q < R::NQ / 2; q++)
+            for (int x = 0; x < 2; x++) {
+                const int k = q + x * R::NQ / 2;
+                cart_words<MODE, DIM>(lo.corner(k * C::STEP), w + 2 * R::W * k);
+            }
+        for (int q = 0; q < R::NQ / 2; q++)
+            for (int x = 0; x < 2; x++) {
+                const int k = q + x * R::NQ / 2;
+                cart_words<MODE, DIM>(hi.corner(k * C::STEP), w + 2 * R::W * k + R::W);
+            }
         if (!last.rows) {
             cart_interp_f32<MODE, DIM>(f, w, tloc, loc, out);
             return;
