@@ -248,6 +248,7 @@ DevField bind_field(fvc_ctx *c, int lo, int hi, double tmin, double tmax) {
     f.tmin = tmin;
     f.tmax = tmax;
     f.vals = c->slice_vals[lo] | c->slice_vals[hi];
+    if (c->edge > 0.0) f.crossings = (float)(std::max(c->slice_speed[lo], c->slice_speed[hi]) / c->edge);
     return f;
 }
 
@@ -482,6 +483,41 @@ static double build_frames(const fvc_mesh_desc *md, const double centre[3], std:
     return *std::max_element(part.begin(), part.end());
 }
 
+/* the k-th of a spread of sample indices below n (multiples of the golden
+ * ratio, so that no stride of the numbering is met) */
+static int64_t spread(int64_t k, int64_t n) {
+    const double g = 0.6180339887498949 * (double)k;
+    return std::min(n - 1, (int64_t)((g - floor(g)) * (double)n));
+}
+
+/* mean element edge, from the volumes of 512 elements */
+static double mean_edge(const fvc_mesh_desc *md) {
+    constexpr int SAMPLE = 512;
+    double sum = 0.0;
+    for (int k = 0; k < SAMPLE; k++) {
+        const int32_t *q = md->conn + 4 * spread(k, md->num_elems);
+        double E[3][3];
+        for (int r = 0; r < md->dims; r++)
+            for (int a = 0; a < 3; a++) E[r][a] = md->coords[3 * (int64_t)q[r + 1] + a] - md->coords[3 * (int64_t)q[0] + a];
+        sum += fabs(md->dims == 2 ? E[0][0] * E[1][1] - E[0][1] * E[1][0]
+                                  : E[0][0] * (E[1][1] * E[2][2] - E[1][2] * E[2][1]) -
+                                        E[0][1] * (E[1][0] * E[2][2] - E[1][2] * E[2][0]) +
+                                        E[0][2] * (E[1][0] * E[2][1] - E[1][1] * E[2][0]));
+    }
+    return pow(sum / SAMPLE, 1.0 / md->dims);
+}
+
+/* rms speed of a slice at 64 of its nodes */
+static double rms_speed(const double *uvw, int64_t n) {
+    constexpr int SAMPLE = 64;
+    double sum = 0.0;
+    for (int k = 0; k < SAMPLE; k++) {
+        const double *v = uvw + 3 * spread(k, n);
+        sum += v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+    }
+    return sqrt(sum / SAMPLE);
+}
+
 /* ------------------------------------------------------------------------ */
 /* context                                                                   */
 /* ------------------------------------------------------------------------ */
@@ -504,6 +540,7 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
     c->slice_scale.assign(pp->max_slices, 1.0f);
     c->slice_time.assign(pp->max_slices, 0.0);
     c->slice_vals.assign(pp->max_slices, VALS_INF | VALS_Z);
+    c->slice_speed.assign(pp->max_slices, 0.0);
     c->sr_slices.assign(pp->max_slices, nullptr);
     memset(&c->mesh, 0, sizeof c->mesh);
     DevMesh &m = c->mesh;
@@ -631,6 +668,7 @@ extern "C" int fvc_create(const fvc_mesh_desc *md, const fvc_params *pp, fvc_ctx
         m.conn = c->conn;
         m.adj = c->adj;
         m.gq = (float)(12.0 * ldexp(1.0, -24) * maxrow);
+        c->edge = mean_edge(md);
         if ((rc = build_hash(c, md))) {
             fvc_destroy(c);
             return rc;
@@ -819,6 +857,7 @@ extern "C" int fvc_load_slice(fvc_ctx *c, int32_t slot, double timestamp, const 
         return set_err(c, FVC_E_HIP, "slice upload");
     c->slice_scale[slot] = scale;
     c->slice_vals[slot] = vals;
+    if (c->mesh.mesh_type == 1) c->slice_speed[slot] = rms_speed(uvw, n);
     c->slice_time[slot] = timestamp;
     return FVC_OK;
 }

@@ -97,7 +97,7 @@ __device__ void batch_particle(const DevMesh &m, const BatchDev &b, int i, int b
     int fl = b.flags[i];
     if (fl & FL_DONE) return;
     const DevRelease R = b.rel[b.rel_id[i]];
-    const bool hist = GEN && (R.itype == INT_AB2 || R.itype == INT_AB3);
+    const bool hist = GEN != 0 && GEN != 3 && (R.itype == INT_AB2 || R.itype == INT_AB3);
     PState s;
     /* V is set at release time and not used again (no extrapolation) */
     for (int c = 0; c < 3; c++) {
@@ -184,7 +184,7 @@ __device__ void batch_particle(const DevMesh &m, const BatchDev &b, int i, int b
     }
 }
 
-/* GEN = 0: RK4 releases only (no multistep state in registers), held to
+/* GEN = 0 and 3: RK4 releases only (no multistep state in registers), held to
  * 3 waves/SIMD (at most 168 VGPRs); 2: AB2 and AB3 releases in the reduced
  * precisions, the same; 1: any others among them, at 2 waves/SIMD (about 235
  * VGPRs, where 3 waves spill 70-87 of them). */
@@ -352,6 +352,7 @@ struct fvc_batch {
     int64_t cls_n0[2];  /* class 0: RK4 releases, class 1: the others */
     int nrel;
     int ab_only; /* class 1 holds AB2 and AB3 releases only */
+    int gen[2];  /* the build (GEN) of each class, chosen by the run for the slices it finds */
     double t0, fdt, dt;
     int nslots;
     int64_t max_budget; /* per-particle bound on budget units for the whole run */
@@ -367,7 +368,7 @@ struct fvc_batch {
      * run so far; kept until the batch is released, so a sweep captures each
      * configuration once and never destroys a graph between runs */
     struct Group {
-        int block, budget, grid0, grid1;
+        int block, budget, grid0, grid1, gen0, gen1;
         hipGraph_t graph;
         hipGraphExec_t exec;
     };
@@ -410,10 +411,11 @@ static bool block_ok(int prec, int bs) {
     return bs == 256;
 }
 
-/* FP64 has no AB build (GEN = 2): the general one takes its place */
+/* FP64 has no AB build (GEN = 2): the general one takes its place; the
+ * reduced precisions have no RK4 by straight walks (GEN = 3) */
 template <int MODE, int GEN>
 constexpr int gen_of() {
-    return MODE == P_F64 && GEN == 2 ? 1 : GEN;
+    return MODE == P_F64 ? (GEN == 2 ? 1 : GEN) : (GEN == 3 ? 0 : GEN);
 }
 
 template <int MODE, int BS, int GEN>
@@ -444,8 +446,11 @@ static int grid_for_batch(fvc_batch *b, int k, int bs, int waves_per_cu) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0)
         cus = 256;
     int blocks_per_cu = 0;
-    const void *fn = !k ? batch_kernel<0>(c->precision, bs)
-                        : b->ab_only ? batch_kernel<2>(c->precision, bs) : batch_kernel<1>(c->precision, bs);
+    const int gen = b->gen[k];
+    const void *fn = gen == 0   ? batch_kernel<0>(c->precision, bs)
+                     : gen == 1 ? batch_kernel<1>(c->precision, bs)
+                     : gen == 2 ? batch_kernel<2>(c->precision, bs)
+                                : batch_kernel<3>(c->precision, bs);
     if (waves_per_cu > 0) {
         blocks_per_cu = std::max(1, waves_per_cu / (bs / 64));
     } else if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks_per_cu, fn, bs, 0) != hipSuccess ||
@@ -458,12 +463,12 @@ static int grid_for_batch(fvc_batch *b, int k, int bs, int waves_per_cu) {
 
 template <int MODE, int BS>
 static void launch_k(fvc_batch *b, int k, int grid, int budget, const BatchDev &d) {
-    if (k && b->ab_only)
-        k_batch<MODE, BS, gen_of<MODE, 2>()><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget);
-    else if (k)
-        k_batch<MODE, BS, 1><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget);
-    else
-        k_batch<MODE, BS, 0><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget);
+    switch (b->gen[k]) {
+    case 0: k_batch<MODE, BS, 0><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget); break;
+    case 2: k_batch<MODE, BS, gen_of<MODE, 2>()><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget); break;
+    case 3: k_batch<MODE, BS, gen_of<MODE, 3>()><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget); break;
+    default: k_batch<MODE, BS, 1><<<grid, BS, 0, b->ctx->stream>>>(b->ctx->mesh, d, budget);
+    }
 }
 
 /* one launch of the sequence for class k: queue reset, batch kernel, compaction */
@@ -699,6 +704,10 @@ extern "C" int fvc_batch_run(fvc_batch *b, const fvc_batch_params *bp, int64_t *
     if (bp->steps_per_launch < 0 || bp->waves_per_cu < 0 || bp->waves_per_cu > 64)
         return set_err(c, FVC_E_INVALID, "batch: steps_per_launch or waves_per_cu out of range");
     const int budget = bp->steps_per_launch == 0 ? 0x7fffffff : bp->steps_per_launch;
+    double crossings = 0.0;
+    for (int k = 0; k < b->nslots && c->edge > 0.0; k++) crossings = std::max(crossings, c->slice_speed[k] / c->edge);
+    b->gen[0] = rk4_walks(c, crossings, b->dt) ? 3 : 0;
+    b->gen[1] = b->ab_only && ab_machine(c, crossings, b->dt, b->fdt, b->cls_n0[1]) ? 2 : 1;
     const int grid[2] = {grid_for_batch(b, 0, bs, bp->waves_per_cu), grid_for_batch(b, 1, bs, bp->waves_per_cu)};
     /* every launch takes at least one budget unit from each active particle */
     const int64_t max_rounds = b->max_budget / std::min<int64_t>(budget, b->max_budget) + 2;
@@ -709,9 +718,11 @@ extern "C" int fvc_batch_run(fvc_batch *b, const fvc_batch_params *bp, int64_t *
     hipGraphExec_t gexec = nullptr;
     if (bp->use_graph) {
         for (const auto &g : b->groups)
-            if (g.block == bs && g.budget == budget && g.grid0 == grid[0] && g.grid1 == grid[1]) gexec = g.exec;
+            if (g.block == bs && g.budget == budget && g.grid0 == grid[0] && g.grid1 == grid[1] &&
+                g.gen0 == b->gen[0] && g.gen1 == b->gen[1])
+                gexec = g.exec;
         if (!gexec) {
-            fvc_batch::Group g{bs, budget, grid[0], grid[1], nullptr, nullptr};
+            fvc_batch::Group g{bs, budget, grid[0], grid[1], b->gen[0], b->gen[1], nullptr, nullptr};
             FVC_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             enqueue_group(b, bs, grid, budget);
             const hipError_t e = hipStreamEndCapture(c->stream, &g.graph);

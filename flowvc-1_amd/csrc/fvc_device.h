@@ -81,6 +81,7 @@ struct DevField {
     double tmin, tmax;
     /* what the FP64 values of the two slices may hold (Cartesian meshes) */
     int vals = VALS_INF | VALS_Z;
+    float crossings = 0.0f; /* for the host's choice of a build: rms speed over the mean element edge */
     /* strain-rate slices at tmin, tmax when the activation potential is integrated, else null */
     const double *sr_lo = nullptr, *sr_hi = nullptr;
     /* exposure time accumulators (per element: 128-bit fixed-point time, encounters), else null */
@@ -1402,11 +1403,19 @@ struct SmRows {
     static constexpr int N = MODE == P_F64 ? NN * DIM : FRAME + VEL; /* FP64: velocities only (rk4_sm64) */
 };
 
-/* rows per lane of the RK4 (GEN = 0) and Adams-Bashforth (GEN = 2) kernels, and this lane's in a block of
+/* GEN, the build of interval_run that a kernel compiles:
+ *   0  RK4 without extrapolation, strain rate or exposure time, with LDS rows:
+ *      rk4_sm, rk4_sm64, rk4_cart
+ *   1  every integrator and option, straight-line walks
+ *   2  AB2 and AB3 without those options on rk4_sm (reduced precision,
+ *      unstructured)
+ *   3  RK4 with straight-line walks (FP64, unstructured)
+ * Where two of them can run, they give the same bits. */
+/* rows per lane of the kernels that have them, and this lane's in a block of
  * BS lanes (null where there are none) */
 template <int MODE, int DIM, int UNS, int GEN>
 constexpr int lane_rows() {
-    return GEN == 1 ? 0 : UNS ? SmRows<MODE, DIM>::N : CartRows<MODE, DIM>::N;
+    return GEN == 1 || GEN == 3 ? 0 : UNS ? SmRows<MODE, DIM>::N : CartRows<MODE, DIM>::N;
 }
 
 template <int MODE, int DIM, int UNS, int GEN, int BS>
@@ -2089,8 +2098,8 @@ __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, ISta
                             int itype_rt, int extrap, int max_steps, int &err, uint32_t &nsteps, double &stop,
                             float4 *rows = nullptr) {
 #pragma clang fp contract(off)
-    /* GEN = 0 compiles RK4 only (no multistep state in registers) */
-    const int itype = GEN ? itype_rt : INT_RK4;
+    /* GEN = 0 and 3 compile RK4 only (no multistep state in registers) */
+    const int itype = GEN == 0 || GEN == 3 ? INT_RK4 : itype_rt;
     if constexpr (MODE == P_F64 && UNSTRUCT && !GEN) {
         if (!extrap) return rk4_sm64<DIM>(m, f, p, is, a, b, dt, max_steps, err, nsteps, stop, rows);
     }
@@ -2142,8 +2151,8 @@ __device__ int interval_run(const DevMesh &m, const DevField &f, PState &p, ISta
     /* activation potential (integration.c:355-360, 449-455): Scalar gains
      * h (S0 + S1) / 2 per step that stays in the domain, S0 and S1 the strain
      * rate at the step's start and end; only the generic integrator build */
-    const bool ap = GEN && f.sr_lo != nullptr;
-    const bool cet = GEN && UNSTRUCT && f.cet_lo != nullptr; /* exposure time (integration.c:427-448) */
+    const bool ap = GEN == 1 && f.sr_lo != nullptr;
+    const bool cet = GEN == 1 && UNSTRUCT && f.cet_lo != nullptr; /* exposure time (integration.c:427-448) */
     using CT = typename VelT<MODE>::T; /* reduced-precision interpolation reads (float) r, s, t */
     CT c_r = 0, c_s = 0, c_t = 0;
     /* Reduced-precision modes on unstructured meshes integrate in FP32: stage

@@ -136,7 +136,7 @@ __device__ __forceinline__ void advect_body(const DevMesh &m, const DevField &f,
         if (!particle_live(p, i, extrap)) {
             idle = true;
         } else {
-            const bool hist = GEN && itype >= 3;
+            const bool hist = (GEN == 1 || GEN == 2) && itype >= 3;
             PState s;
             load_state(p, i, s, hist, extrap);
             int err = 0;
@@ -179,12 +179,19 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_GEN_W
 /* AB2 and AB3 of the reduced-precision modes on unstructured meshes, without
  * strain rate, exposure time or extrapolation (k_advect_gen takes the rest):
  * the state machine, 3 waves per SIMD */
-template <int MODE, int DIM, int UNS>
+template <int MODE, int DIM>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void k_advect_ab(
     DevMesh m, DevField f, PtrSet p, const int *__restrict__ index, int64_t begin, int64_t count, double t1, double t2,
     int itype, double dt, ErrBuf eb, unsigned long long *steps) {
-    if constexpr (UNS && MODE != P_F64)
-        advect_body<MODE, DIM, UNS, 2>(m, f, p, index, begin, count, t1, t2, itype, dt, 0, eb, steps);
+    advect_body<MODE, DIM, 1, 2>(m, f, p, index, begin, count, t1, t2, itype, dt, 0, eb, steps);
+}
+
+/* FP64 RK4 on unstructured meshes by straight-line walks (rk4_walks) */
+template <int DIM>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_HOT_WAVES))) void k_advect_walk(
+    DevMesh m, DevField f, PtrSet p, const int *__restrict__ index, int64_t begin, int64_t count, double t1, double t2,
+    double dt, ErrBuf eb, unsigned long long *steps) {
+    advect_body<P_F64, DIM, 1, 3>(m, f, p, index, begin, count, t1, t2, INT_RK4, dt, 0, eb, steps);
 }
 
 /* Each particle over its own segment: tt[2q], tt[2q+1] = t1, t2 of particle
@@ -199,7 +206,7 @@ __device__ __forceinline__ void k_advect_times_body(const DevMesh &m, const DevF
         const double t1 = tt[2 * q], t2 = tt[2 * q + 1];
         const int64_t i = begin + q;
         if (t1 == t1 && p.left_time[i] > -TINY && (!p.left[i] || extrap)) {
-            const bool hist = GEN && itype >= 3;
+            const bool hist = (GEN == 1 || GEN == 2) && itype >= 3;
             PState s;
             load_state(p, i, s, hist, extrap);
             int err = 0;
@@ -233,6 +240,30 @@ __global__ __launch_bounds__(BLOCK) void k_launch_vel(DevMesh m, DevField f, Ptr
     for (int c = 0; c < 3; c++) s.V[c] = v[c];
     store_state(p, i, s);
 }
+
+#define FVC_DISPATCH_DIM(DIM_, KERNEL, ...)                                                                            \
+    do {                                                                                                               \
+        if (DIM_ == 3) KERNEL<3> __VA_ARGS__;                                                                          \
+        else KERNEL<2> __VA_ARGS__;                                                                                    \
+    } while (0)
+
+/* the reduced precisions on unstructured meshes */
+#define FVC_DISPATCH_REDUCED(MODE_, DIM_, KERNEL, ...)                                                                 \
+    do {                                                                                                               \
+        if (DIM_ == 3) {                                                                                               \
+            switch (MODE_) {                                                                                           \
+            case P_F32: KERNEL<P_F32, 3> __VA_ARGS__; break;                                                           \
+            case P_BF16: KERNEL<P_BF16, 3> __VA_ARGS__; break;                                                         \
+            default: KERNEL<P_F16, 3> __VA_ARGS__; break;                                                              \
+            }                                                                                                          \
+        } else {                                                                                                       \
+            switch (MODE_) {                                                                                           \
+            case P_F32: KERNEL<P_F32, 2> __VA_ARGS__; break;                                                           \
+            case P_BF16: KERNEL<P_BF16, 2> __VA_ARGS__; break;                                                         \
+            default: KERNEL<P_F16, 2> __VA_ARGS__; break;                                                              \
+            }                                                                                                          \
+        }                                                                                                              \
+    } while (0)
 
 #define FVC_DISPATCH(MODE_, DIM_, UNS_, KERNEL, ...)                                                                   \
     do {                                                                                                               \
@@ -297,6 +328,14 @@ int launch_velocity(fvc_ctx *c, PtrSet p, int64_t begin, int64_t count, double t
     return check_err(c, "fvc_launch_velocity");
 }
 
+/* FP64 RK4 on unstructured meshes by straight-line walks (rk4_walks) */
+template <int DIM>
+__global__ __launch_bounds__(BLOCK) void k_advect_times_walk(DevMesh m, DevField f, PtrSet p, int64_t begin,
+                                                            int64_t count, const double *__restrict__ tt, double dt,
+                                                            int extrap, ErrBuf eb, unsigned long long *steps) {
+    k_advect_times_body<P_F64, DIM, 1, 3>(m, f, p, begin, count, tt, INT_RK4, dt, extrap, eb, steps);
+}
+
 template <int MODE, int DIM, int UNS>
 __global__ __launch_bounds__(BLOCK) void k_advect_times_rk4(DevMesh m, DevField f, PtrSet p, int64_t begin,
                                                            int64_t count, const double *__restrict__ tt, int itype,
@@ -309,7 +348,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_GEN_W
 int launch_advect_times(fvc_ctx *c, PtrSet p, int64_t begin, int64_t count, const double *dtt, const DevField &f,
                         const fvc_int_params &ip) {
     if (count > 0) {
-        if (ip.int_type == FVC_INT_RK4 && !f.sr_lo && !f.cet_lo)
+        if (ip.int_type == FVC_INT_RK4 && !f.sr_lo && !f.cet_lo && rk4_walks(c, f.crossings, ip.time_step))
+            FVC_DISPATCH_DIM(c->mesh.dims, k_advect_times_walk,
+                             <<<grid_for(count, BLOCK), BLOCK, 0, c->stream>>>(c->mesh, f, p, begin, count, dtt,
+                                                                               ip.time_step, ip.extrapolate, errbuf(c),
+                                                                               c->d_steps));
+        else if (ip.int_type == FVC_INT_RK4 && !f.sr_lo && !f.cet_lo)
             FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_advect_times_rk4,
                          <<<grid_for(count, BLOCK), BLOCK, 0, c->stream>>>(c->mesh, f, p, begin, count, dtt,
                                                                            ip.int_type, ip.time_step, ip.extrapolate,
@@ -366,17 +410,24 @@ int launch_advect(fvc_ctx *c, PtrSet p, const int *index, int64_t begin, int64_t
         if (block != BLOCK) block = BLOCK; /* kernels are compiled for 256-lane blocks */
         timing_begin(c);
         /* strain rate, exposure, extrapolation: generic build only */
-        if (ip.int_type == FVC_INT_RK4 && !ip.extrapolate && !f.sr_lo && !f.cet_lo)
+        const bool plain = !ip.extrapolate && !f.sr_lo && !f.cet_lo;
+        if (ip.int_type == FVC_INT_RK4 && plain && rk4_walks(c, f.crossings, ip.time_step))
+            FVC_DISPATCH_DIM(c->mesh.dims, k_advect_walk,
+                             <<<grid_for(count, block), block, 0, c->stream>>>(c->mesh, f, p, index, begin, count, t1,
+                                                                               t2, ip.time_step, errbuf(c),
+                                                                               c->d_steps));
+        else if (ip.int_type == FVC_INT_RK4 && plain)
             FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_advect,
                          <<<grid_for(count, block), block, 0, c->stream>>>(c->mesh, f, p, index, begin, count, t1, t2,
                                                                            ip.int_type, ip.time_step, ip.extrapolate,
                                                                            errbuf(c), c->d_steps));
         else if ((ip.int_type == FVC_INT_AB2 || ip.int_type == FVC_INT_AB3) && c->mesh.mesh_type == 1 &&
-                 c->precision != FVC_PREC_F64 && !ip.extrapolate && !f.sr_lo && !f.cet_lo)
-            FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_advect_ab,
-                         <<<grid_for(count, block), block, 0, c->stream>>>(c->mesh, f, p, index, begin, count, t1, t2,
-                                                                           ip.int_type, ip.time_step, errbuf(c),
-                                                                           c->d_steps));
+                 c->precision != FVC_PREC_F64 && plain &&
+                 ab_machine(c, f.crossings, ip.time_step, t2 - t1, count))
+            FVC_DISPATCH_REDUCED(c->precision, c->mesh.dims, k_advect_ab,
+                                 <<<grid_for(count, block), block, 0, c->stream>>>(c->mesh, f, p, index, begin, count,
+                                                                                   t1, t2, ip.int_type, ip.time_step,
+                                                                                   errbuf(c), c->d_steps));
         else
             FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_advect_gen,
                          <<<grid_for(count, block), block, 0, c->stream>>>(c->mesh, f, p, index, begin, count, t1, t2,
@@ -1331,6 +1382,14 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_RK4_W
     ftle_advect_body<MODE, DIM, UNS, 0>(m, f, d, active, nactive, t1, t2, itype, dt, 0, eb, steps);
 }
 
+/* FP64 RK4 on unstructured meshes by straight-line walks (rk4_walks) */
+template <int DIM>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_HOT_WAVES))) void k_ftle_advect_walk(
+    DevMesh m, DevField f, FtleDev d, const int *__restrict__ active, int64_t nactive, double t1, double t2, double dt,
+    ErrBuf eb, unsigned long long *steps) {
+    ftle_advect_body<P_F64, DIM, 1, 3>(m, f, d, active, nactive, t1, t2, INT_RK4, dt, 0, eb, steps);
+}
+
 template <int MODE, int DIM, int UNS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(FVC_GEN_WAVES(MODE)))) void k_ftle_advect_gen(DevMesh m, DevField f, FtleDev d,
                                                           const int *__restrict__ active, int64_t nactive, double t1,
@@ -1642,19 +1701,28 @@ __device__ __forceinline__ void early_body(const DevMesh &m, const DevField &f, 
     }
 }
 
+/* The RK4 build of the early FTLE.  In FP64 on unstructured meshes the
+ * straight-line walks: a few lanes of a wave integrate, one element's
+ * geometry after the other, and the state machine, 0.9-1.1 times as fast at
+ * 0.1 elements a step and fewer, was 0.55-0.75 from 0.2 on. */
+template <int MODE, int UNS>
+constexpr int early_gen() {
+    return MODE == P_F64 && UNS ? 3 : 0;
+}
+
 /* RK4 frames, live input: the frame's points when it has more than `above` */
 template <int MODE, int DIM, int UNS>
 __global__ __launch_bounds__(BLOCK) void k_early(DevMesh m, DevField f, FtleDev d, const int *__restrict__ list,
                                                 const int *__restrict__ d_nt, int64_t above, double t1, int itype,
                                                 double dt, ErrBuf eb) {
-    early_body<MODE, DIM, UNS, 0, 0>(m, f, d, list, d_nt, EarlySnap{}, above, t1, itype, dt, eb);
+    early_body<MODE, DIM, UNS, early_gen<MODE, UNS>(), 0>(m, f, d, list, d_nt, EarlySnap{}, above, t1, itype, dt, eb);
 }
 
 /* RK4 frames, from the stencil snapshot (at most cap triggered points) */
 template <int MODE, int DIM, int UNS>
 __global__ __launch_bounds__(BLOCK) void k_early_snapped(DevMesh m, DevField f, FtleDev d, EarlySnap sn, double t1,
                                                         int itype, double dt, ErrBuf eb) {
-    early_body<MODE, DIM, UNS, 0, 1>(m, f, d, nullptr, nullptr, sn, 0, t1, itype, dt, eb);
+    early_body<MODE, DIM, UNS, early_gen<MODE, UNS>(), 1>(m, f, d, nullptr, nullptr, sn, 0, t1, itype, dt, eb);
 }
 
 /* Euler frames */
@@ -1889,7 +1957,12 @@ int launch_ftle_frame(fvc_ftle *f, int lo, int hi, double tmin, double tmax, dou
     }
     if (f->nactive > 0) {
         timing_begin(c);
-        if (itype == 1 && !ip.extrapolate)
+        if (itype == INT_RK4 && !ip.extrapolate && rk4_walks(c, fld.crossings, ip.time_step))
+            FVC_DISPATCH_DIM(c->mesh.dims, k_ftle_advect_walk,
+                             <<<grid_for(f->nactive, BLOCK), BLOCK, 0, c->stream>>>(c->mesh, fld, d, f->active,
+                                                                                    f->nactive, t1, t2, ip.time_step,
+                                                                                    errbuf(c), c->d_steps));
+        else if (itype == INT_RK4 && !ip.extrapolate)
             FVC_DISPATCH(c->precision, c->mesh.dims, c->mesh.mesh_type, k_ftle_advect,
                          <<<grid_for(f->nactive, BLOCK), BLOCK, 0, c->stream>>>(c->mesh, fld, d, f->active,
                                                                                 f->nactive, t1, t2, itype,

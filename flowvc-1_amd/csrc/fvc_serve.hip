@@ -103,7 +103,7 @@ __device__ uint32_t serve_particle(const DevMesh &m, const SrvDev &S, int i, int
     r_out = r;
     const SrvReq R = S.req[r];
     const bool ftle = R.kind == FVC_REQ_FTLE;
-    const bool hist = GEN && !ftle && (R.itype == INT_AB2 || R.itype == INT_AB3);
+    const bool hist = GEN == 1 && !ftle && (R.itype == INT_AB2 || R.itype == INT_AB3);
     const bool started = (fl & SF_STARTED) != 0;
     PState s;
     for (int c = 0; c < 3; c++) {
@@ -213,7 +213,7 @@ __device__ uint32_t serve_particle(const DevMesh &m, const SrvDev &S, int i, int
 /* GEN = 0: RK4 requests (tracer or FTLE), 3 waves/SIMD; 1: the other
  * integrators, 2 waves/SIMD (no spills; 3 waves spill 70 VGPRs) */
 template <int MODE, int BS, int GEN>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(GEN ? 2 : FVC_HOT_WAVES))) void k_serve(DevMesh m, SrvDev S,
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(GEN == 1 ? 2 : FVC_HOT_WAVES))) void k_serve(DevMesh m, SrvDev S,
                                                                                       int budget) {
     const int lane = threadIdx.x & 63;
     const int home = blockIdx.x % NQ;
@@ -505,6 +505,7 @@ struct fvc_server {
     int cur; /* parity of the list the next launch reads */
     int grid[2];
     hipGraphExec_t gexec[2];
+    bool walks = false; /* FP64: RK4 requests by straight-line walks (rk4_walks) */
     hipGraph_t graph[2];
     /* host bookkeeping */
     std::map<int64_t, int64_t> free_ranges; /* base -> length */
@@ -559,8 +560,11 @@ static SrvDev srv_dev(fvc_server *S, int k, int parity) {
 
 template <int MODE, int BS>
 static void launch_serve(fvc_server *S, int k, int grid, const SrvDev &d, int budget) {
+    constexpr int WALK = MODE == P_F64 ? 3 : 0;
     if (k)
         k_serve<MODE, BS, 1><<<grid, BS, 0, S->ctx->stream>>>(S->ctx->mesh, d, budget);
+    else if (S->walks)
+        k_serve<MODE, BS, WALK><<<grid, BS, 0, S->ctx->stream>>>(S->ctx->mesh, d, budget);
     else
         k_serve<MODE, BS, 0><<<grid, BS, 0, S->ctx->stream>>>(S->ctx->mesh, d, budget);
 }
@@ -570,9 +574,10 @@ static const void *serve_fn() {
     return reinterpret_cast<const void *>(&k_serve<MODE, BS, GEN>);
 }
 
-static const void *serve_kernel(int prec, int bs, int k) {
+static const void *serve_kernel(int prec, int bs, int k, bool walks) {
     switch (prec) {
-    case FVC_PREC_F64: return k ? serve_fn<P_F64, 256, 1>() : serve_fn<P_F64, 256, 0>();
+    case FVC_PREC_F64:
+        return k ? serve_fn<P_F64, 256, 1>() : walks ? serve_fn<P_F64, 256, 3>() : serve_fn<P_F64, 256, 0>();
     case FVC_PREC_BF16: return k ? serve_fn<P_BF16, 256, 1>() : serve_fn<P_BF16, 256, 0>();
     case FVC_PREC_F16: return k ? serve_fn<P_F16, 256, 1>() : serve_fn<P_F16, 256, 0>();
     default:
@@ -964,9 +969,12 @@ extern "C" int fvc_server_create(fvc_ctx *c, const fvc_server_params *sp_in, fvc
         fvc_server_destroy(S);
         return srv_err(c, FVC_E_HIP, "server init");
     }
+    /* by the slices resident now (the graphs below keep the choice) */
+    for (int k = 0; k < sp.nslots && c->edge > 0.0; k++)
+        S->walks = S->walks || rk4_walks(c, c->slice_speed[k] / c->edge, sp.time_step);
     for (int kk = 0; kk < 2; kk++) {
         int bpc = 0;
-        const void *fn = serve_kernel(c->precision, sp.block, kk);
+        const void *fn = serve_kernel(c->precision, sp.block, kk, S->walks);
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0)
             cus = 256;
