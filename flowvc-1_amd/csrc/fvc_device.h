@@ -1388,8 +1388,8 @@ enum { PH_F0 = 0, PH_K2 = 1, PH_K3 = 2, PH_K4 = 3, PH_LOC = 4, PH_DONE = 5 };
  * cycles (1.1-1.2 look-ups per CU and cycle, 32 per particle-step) with the
  * vector ALUs at 64-68%; but a probe moves a tenth of an element per step, so
  * nearly every pass asks for what the lane had in the pass before.  With the
- * rows only lanes whose element changed gather: 5.8 look-ups per step, vector
- * ALUs 72-79% busy.  k_advect (4M tracers, 20 steps, 5.6M tets) 3.44 -> 2.76
+ * rows only lanes whose element changed gather: 5.1-5.5 look-ups per step,
+ * vector ALUs 77-80% busy.  k_advect (4M tracers, 20 steps, 5.6M tets) 3.44 -> 2.76
  * ms a launch, k_ftle_advect (96x96x480 points) 4.49 -> 2.66 ms, the RK4
  * class of a batch 2.1 -> 1.2 ms.  LDS and not registers: held in registers
  * (40 more) the kernels spill 56-64 at 4 waves per SIMD.  160 bytes a lane
@@ -1532,6 +1532,7 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
         }
         gc = guard_offset(m, c);
     };
+    const int order = itype == INT_AB2 ? 2 : 3;
     /* start of a step (the loop head of integration.c:344); false when the
      * interval is done or the step budget spent */
     auto begin_step = [&]() -> bool {
@@ -1549,11 +1550,14 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
         tlh = (float)((is.tc + is.h / 2 - f.tmin) * inv_span); /* lies between l0 and l1 */
         tl1 = (float)l1;
         if ((l0 > 1 + TINY) || (l0 < 0 - TINY)) err = E_TLOC;
-        /* only RK4 steps read the field at their end: AB tests l1 where it knows */
-        if (!AB && ((l1 > 1 + TINY) || (l1 < 0 - TINY))) err = E_TLOC;
+        if (AB) {
+            const bool micro = fabs(is.h) <= hmin, full = fabs(is.h - hfull) <= 1e-9 * fabs(hfull);
+            multi = micro || (full && p.nhist >= order - 1);
+        }
+        /* only RK4 steps read the field at their end */
+        if (!(AB && multi) && ((l1 > 1 + TINY) || (l1 < 0 - TINY))) err = E_TLOC;
         return true;
     };
-    const int order = itype == INT_AB2 ? 2 : 3;
     /* the increment of a step that is not RK4 */
     auto multi_inc = [&](double inc[3]) {
         const double h = is.h;
@@ -1693,14 +1697,7 @@ __device__ int rk4_sm(const DevMesh &m, const DevField &f, PState &p, IState &is
         }
         if (AB && phase == PH_F0) {
             for (int k3 = 0; k3 < 3; k3++) f0[k3] = k[k3];
-            const bool micro = fabs(is.h) <= hmin, full = fabs(is.h - hfull) <= 1e-9 * fabs(hfull);
-            multi = micro || (full && p.nhist >= order - 1);
             if (!multi) {
-                const double l1 = (is.tc + is.h - f.tmin) * inv_span;
-                if ((l1 > 1 + TINY) || (l1 < 0 - TINY)) {
-                    err = E_TLOC;
-                    break;
-                }
                 anchor();
             } else { /* on to the locate walk, the ring back at the first stage */
                 const int last = q3;
