@@ -39,7 +39,7 @@ struct fvc_ctx {
     std::vector<void *> slices;
     std::vector<float> slice_scale;
     std::vector<double> slice_time;
-    std::vector<int> slice_vals; /* Cartesian meshes: VALS_* of each slice */
+    std::vector<int> slice_vals; /* VALS_* of each slice, looked at for 2-D grids in FP64 */
     std::vector<double> slice_speed; /* unstructured meshes: rms speed of each slice, by a sample of its nodes */
     double edge = 0.0;  /* unstructured meshes: mean element edge, by a sample of the elements */
     int64_t nvel;       /* nodes per slice */
@@ -59,7 +59,7 @@ struct fvc_ctx {
     unsigned long long *d_steps;
     unsigned long long steps_seen[2]; /* steps[0], steps[1] when last taken */
     int64_t last_steps;
-    int64_t last_idle; /* lanes of the last fvc_advect launch whose particle was not integrated */
+    int64_t last_idle; /* lanes of the last fvc_advect or fvc_ftle_frame launch whose particle was not integrated */
     std::string last_error;
     int64_t bytes_used;
     /* scratch (grown on demand) */
