@@ -119,6 +119,39 @@ def test_stenosis2d_frames_within_first_order_bound():
     assert (err <= bound).all(), float((err / bound).max())
 
 
+def test_location_far_from_the_element_within_first_order_bound():
+    """Location and its walks form the query from the FP64 difference to the
+    frame's origin, rounded once, and meet elements the query is far from: up
+    to 1,000 elements away the error stays below (18 cond + 12) 2^-24 L, L the
+    largest natural coordinate."""
+    P, conn = _pipe()
+    Minv, M, o, lo, cond, _ = frames(P, conn, 3)
+    rng = np.random.default_rng(5)
+    n = 200_000
+    e = rng.integers(0, conn.shape[0], n)
+    lam = queries(rng, n, 3)
+    lam[n // 2:, 1:] *= 10.0 ** rng.uniform(0.0, 3.0, (n - n // 2, 1))
+    P0 = P[conn[e, 0]]
+    E = np.stack([P[conn[e, q + 1]] - P0 for q in range(3)], axis=2)
+    X = P0 + np.einsum("nij,nj->ni", E, lam[:, 1:])
+    ex = np.einsum("nij,nj->ni", Minv[e], X - P0)
+    ex = np.concatenate([ex, (1.0 - ex.sum(1))[:, None]], 1)
+    q = (X - o[e].astype(np.float64)).astype(F32)
+    got = []
+    for i in range(3):
+        v = lo[e][:, i]
+        for j in range(3):
+            v = fma(M[e][:, i, j], q[:, j], v)
+        got.append(v)
+    l0 = F32(1) - got[0]
+    for v in got[1:]:
+        l0 = (l0 - v).astype(F32)
+    err = np.abs(np.stack(got + [l0], 1).astype(np.float64) - ex).max(1)
+    L = np.maximum(1.0, np.abs(ex).max(1))
+    assert L.max() > 500
+    assert (err <= (18.0 * cond[e] + 12.0) * U * L).all()
+
+
 def _long_pipe():
     """a pipe 100 long with cells about 0.25 wide: node rounding at the domain's
     extent (2^-24 x 50) is large beside the elements' own rounding (397

@@ -105,14 +105,43 @@ def test_points_too_far_for_a_finite_quotient_are_outside(dims, res, precision):
 REL = {"f32": 20 * 2.0**-24, "bf16": 2.0**-9, "f16": 2.0**-12}
 
 
+def _steady(dims, res, sl, recs, ref, dt, t1, t2, by):
+    """Points whose FP64 exit does not change when they start `by` further
+    along any axis (inwards from where that would leave the grid): none of
+    their walls is so near that an error of that size could decide it."""
+    same = np.ones(recs.size, bool)
+    om = oracle.Mesh(dims, [0.0, 1.0, 0.0, 1.0, 0.0, 1.0 if dims == 3 else 0.0], cart_min=[0.0] * 3,
+                     cart_max=[1.0, 1.0, 1.0 if dims == 3 else 0.0], cart_res=res)
+    for s in range(2):
+        om.set_slot(s, sl[s])
+    om.set_interval(0.0, 1.0)
+    for a in range(dims):
+        for d in (by, -by):
+            r = recs.copy()
+            x = r["X"][:, a] + d
+            r["X"][:, a] = np.where((x < 0.0) | (x > 1.0), r["X"][:, a] - d, x)
+            assert om.advect(r, t1, t2, dt) == 0
+            same &= (r["LeftDomain"] == ref["LeftDomain"]) & (np.abs(r["LeftDomainTime"] - ref["LeftDomainTime"]) < 1.5 * dt)
+    return same
+
+
 @pytest.mark.parametrize("dims,res", [(2, [2, 2, 1]), (2, [37, 18, 1]), (3, [2, 3, 2]), (3, [19, 14, 23])])
 @pytest.mark.parametrize("precision", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("n", [1, 65, 3000])
 def test_reduced_precision_follows_the_oracle(dims, res, precision, n):
     recs = _points(dims, res, 1.0, n, 5)
-    got, ref = _both(dims, res, 1.0, _grid(dims, res, 1.0), recs, precision, 0.01, 0.0, 0.31)
+    sl = _grid(dims, res, 1.0)
+    got, ref = _both(dims, res, 1.0, sl, recs, precision, 0.01, 0.0, 0.31)
     tol = REL[precision] * 1.1 * 0.31 * np.exp(5 * 0.31)
     stay = (got["LeftDomain"] == 0) & (ref["LeftDomain"] == 0)
     assert np.abs(got["X"][stay] - ref["X"][stay]).max(initial=0.0) <= tol
     # an exit may differ where a point comes within tol of a wall (or starts on one)
     assert (got["LeftDomain"] != ref["LeftDomain"]).sum() <= 1 + n * (0.1 + tol / 0.05)
+    # and nowhere else: the points on the wall x = 1 and on the nodes among them
+    sure = _steady(dims, res, sl, recs, ref, 0.01, 0.0, 0.31, 2 * tol)
+    np.testing.assert_array_equal(got["LeftDomain"][sure], ref["LeftDomain"][sure])
+    out = sure & (ref["LeftDomain"] != 0)
+    assert np.abs(got["LeftDomainTime"][out] - ref["LeftDomainTime"][out]).max(initial=0.0) < 1.5 * 0.01
+    if n == 3000:
+        wall = recs["X"][:, 0] == 1.0
+        assert sure.mean() > 0.5 and (sure & wall).sum() > 20 and (sure & stay).sum() > 500 and out.sum() > 100

@@ -72,11 +72,11 @@ def _grade(p):
 
 
 @pytest.mark.parametrize("shape", ["stretched", "graded"])
-@pytest.mark.parametrize("precision", ["f32", "bf16"])
+@pytest.mark.parametrize("precision", ["f64", "f32", "bf16"])
 def test_locate_bit_exact_on_badly_shaped_meshes(pipe, shape, precision):
     """The FP32 frames carry each element's own guard band, set by its
-    condition number: on flat and strongly graded tets the reduced-precision
-    walks must still return the FP64 walk's element for every probe (faces,
+    condition number: on flat and strongly graded tets the walks (location
+    asks the frames first in FP64 too) must still return the FP64 walk's element for every probe (faces,
     edges and vertices included: the probes are mapped like the nodes)."""
     t, xyz, conn, adj, _ = pipe
     f = _stretch if shape == "stretched" else _grade
