@@ -93,8 +93,9 @@ def roofline_valu(kernel, steps_per_launch, avg_ms, bpp, default_workload):
     particle-step (SQ_ACTIVE_INST_VALU x 4 over the particle-steps of the
     profiled launches) x particle-steps of this launch / its measured
     duration, against 1024 SIMDs x 2.4 GHz.  The algorithmic gather bytes
-    (704 B per particle-step in FP32) are reported beside it with the
-    measured HBM traffic (cache-served: their HBM fraction exceeds 1)."""
+    (704 B per particle-step in FP32, as if every test met a new element;
+    most are read from the lanes' LDS rows) are reported beside it with the
+    measured HBM traffic (their HBM fraction exceeds 1)."""
     cyc = profile_figure("pmc_valu_pipe.md", "valu_cycles_per_particle_step", kernel) if default_workload else None
     secs = avg_ms * 1e-3
     gather = steps_per_launch * bpp / secs if secs > 0 else 0.0
