@@ -141,7 +141,7 @@ typedef struct fvc_ftle fvc_ftle;
  * Host memory: 256 KB of pinned memory; outputs over that (fvc_particles_get,
  * fvc_ftle_output, ...) stage through up to 8 MB more, allocated when first
  * needed and held until fvc_destroy, or through the 256 KB where it cannot be
- * had. */
+ * had.  fvc_locate keeps up to 32 MB of device memory (32 B a query point). */
 int fvc_create(const fvc_mesh_desc *mesh, const fvc_params *params, fvc_ctx **out);
 /* Frees the context; objects still alive on it are released and detached
  * (see Lifetimes above). */
